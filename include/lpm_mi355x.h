@@ -185,6 +185,13 @@ int64_t lpm_size(const lpm_ctx *ctx, const char *what);
  *                        coarse correction, SpMV) into a HIP graph and replay it for every batch
  *                        of every solve; re-captured when sizes, launch configuration or buffers
  *                        change. Per-SpMV timing is off in this mode | 0 (default): launch directly
+ *  "cg_persist"       1 (default): systems of up to 131,072 particles run each CG solve in one
+ *                        persistent launch (the same recurrence, stopping rule and precision) |
+ *                        0: one launch per step of every iteration. Launched solves are also
+ *                        kept under cg_graph, spmv_tune = 0 (the caller fixes the SpMV launch) and
+ *                        per-SpMV timing. lpm_stat("cg_persistent") counts the persistent solves
+ *  "cg_wait_ms"       longest wait between workgroups inside a persistent solve (0..60000, default
+ *                        2000); a solve that exceeds it is repeated with launches
  *  "cg_batch"         CG iterations issued before the host reads the device's stop flag (rounded
  *                        up to even; default 16); iterations issued past the stop are no-ops, so
  *                        the batch sizes never change results

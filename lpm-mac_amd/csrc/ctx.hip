@@ -931,6 +931,7 @@ int lpm_destroy(lpm_ctx *c) {
         if (p) hipFree(p);
     dump_free(c);
     coarse_free(c);
+    pcg_free(c);
     fd_free(c);
     fat_record_clear(c);
     for (void *p : c->ckpt)
@@ -1013,6 +1014,11 @@ int lpm_set_mode(lpm_ctx *c, const char *name, double v) {
     else if (w == "cg_forcing") c->cg_forcing = (int)v ? 1 : 0;
     else if (w == "coarse_graph") c->coarse_graph = (int)v ? 1 : 0;
     else if (w == "cg_graph") c->cg_graph = (int)v ? 1 : 0;
+    else if (w == "cg_persist") c->cg_persist = (int)v ? 1 : 0;
+    else if (w == "cg_wait_ms") {
+        if (!(v >= 0 && v <= 60000)) return lpm_fail(c, LPM_E_ARG, "cg_wait_ms must be 0..60000");
+        c->cg_wait_ms = v;
+    }
     else if (w == "coarse_reuse") c->coarse_reuse = (int)v ? 1 : 0;
     else if (w == "coarse_rebuild") {
         if ((int)v) c->coarse_stale = true;  // the next assembly rebuilds the coarse space
@@ -1075,6 +1081,8 @@ double lpm_get_mode(const lpm_ctx *c, const char *name) {
     if (w == "cg_forcing") return c->cg_forcing;
     if (w == "coarse_graph") return c->coarse_graph;
     if (w == "cg_graph") return c->cg_graph;
+    if (w == "cg_persist") return c->cg_persist;
+    if (w == "cg_wait_ms") return c->cg_wait_ms;
     if (w == "coarse_reuse") return c->coarse_reuse;
     if (w == "predictor") return c->predictor;
     if (w == "coarse_cells") return c->coarse_cells;
@@ -1380,6 +1388,7 @@ double lpm_stat(const lpm_ctx *c, const char *name) {
     if (w == "cg_iters") return (double)c->st_cg_iters;
     if (w == "coarse_builds") return (double)c->st_coarse_builds;
     if (w == "cg_solves") return (double)c->st_cg_solves;
+    if (w == "cg_persistent") return (double)c->st_pcg;
     if (w == "assemblies") return (double)c->st_asm;
     if (w == "spmv_launches") return (double)c->st_spmv;
     if (w == "spmv_ms") return c->st_spmv_ms;
@@ -1394,7 +1403,7 @@ double lpm_stat(const lpm_ctx *c, const char *name) {
 int lpm_reset_stats(lpm_ctx *c) {
     if (!c) return LPM_E_ARG;
     c->st_newton = c->st_cg_iters = c->st_cg_solves = c->st_asm = c->st_spmv = c->st_spmv_timed = 0;
-    c->st_coarse_builds = 0;
+    c->st_coarse_builds = c->st_pcg = 0;
     c->st_spmv_ms = 0;
     return LPM_OK;
 }

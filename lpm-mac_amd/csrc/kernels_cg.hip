@@ -883,6 +883,18 @@ static int cg_graph_prepare(lpm_ctx *c, int gv, int gs, int batch, F issue) {
     return LPM_OK;
 }
 
+// what a finished solve left in h_scal, as Eigen reports it
+static void cg_result(lpm_ctx *c, int *iters, double *error, int *success) {
+    const double rhs2 = c->h_scal[SC_RHS2];
+    const double done = c->h_scal[SC_DONE];
+    // Eigen reports the updates done before the converging one (its loop breaks before i++)
+    const int64_t upd = (int64_t)c->h_scal[SC_ITER];
+    if (c->cg_slot >= 0 && c->cg_slot < 4) c->cg_hist[c->cg_slot] = (int)std::min<int64_t>(upd, 1 << 20);
+    *iters = (int)((done == 1.0 && upd > 0) ? upd - 1 : upd);
+    *error = (done == 3.0) ? 0.0 : sqrt(c->h_scal[SC_RR] / rhs2);
+    *success = (done == 3.0) || (*error <= c->cg_tol);
+}
+
 template <typename T, int D, int VP>
 static int cg_t(lpm_ctx *c, int *iters, double *error, int *success) {
     typedef Vec<T, VP> V;
@@ -991,14 +1003,7 @@ static int cg_t(lpm_ctx *c, int *iters, double *error, int *success) {
         if (it0 > maxit + 2 * batch_max) break;  // the device cap stops earlier; this only guards the loop
     }
     c->st_spmv += 1;  // the prologue SpMV
-    const double rhs2 = c->h_scal[SC_RHS2];
-    const double done = c->h_scal[SC_DONE];
-    // Eigen reports the updates done before the converging one (its loop breaks before i++)
-    const int64_t upd = (int64_t)c->h_scal[SC_ITER];
-    if (slot >= 0 && slot < 4) c->cg_hist[slot] = (int)std::min<int64_t>(upd, 1 << 20);
-    *iters = (int)((done == 1.0 && upd > 0) ? upd - 1 : upd);
-    *error = (done == 3.0) ? 0.0 : sqrt(c->h_scal[SC_RR] / rhs2);
-    *success = (done == 3.0) || (*error <= c->cg_tol);
+    cg_result(c, iters, error, success);
     return LPM_OK;
 }
 
@@ -1007,11 +1012,19 @@ int cg_solve(lpm_ctx *c, int *iters, double *error, int *success) {
     int rc = launch_precond_setup(c);
     if (rc) return rc;
     if ((rc = coarse_prepare(c))) return rc;
-    if ((rc = spmv_tune(c))) return rc;
-    if (c->precision == 0)
-        rc = c->dim == 3 ? cg_t<float, 3, 3>(c, iters, error, success) : cg_t<float, 2, 2>(c, iters, error, success);
-    else
-        rc = c->dim == 3 ? cg_t<double, 3, 3>(c, iters, error, success) : cg_t<double, 2, 2>(c, iters, error, success);
+    bool ran = false;
+    if ((rc = pcg_solve(c, c->cg_maxit < 0 ? 2 * c->n * c->dim : c->cg_maxit, &ran))) return rc;
+    if (ran) {
+        c->st_pcg++;
+        c->st_spmv += (int64_t)c->h_scal[SC_ITER];  // one per update
+        cg_result(c, iters, error, success);
+    } else {
+        if ((rc = spmv_tune(c))) return rc;
+        if (c->precision == 0)
+            rc = c->dim == 3 ? cg_t<float, 3, 3>(c, iters, error, success) : cg_t<float, 2, 2>(c, iters, error, success);
+        else
+            rc = c->dim == 3 ? cg_t<double, 3, 3>(c, iters, error, success) : cg_t<double, 2, 2>(c, iters, error, success);
+    }
     if (!rc && two_level(c) && c->coarse_reuse) {
         // a kept coarse space is rebuilt before the next solve once the CG needs clearly more
         // iterations than the first solve after the last build

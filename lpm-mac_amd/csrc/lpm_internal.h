@@ -36,6 +36,7 @@ enum {
     SC_ALPHA_P = SC_GAMMA_P + 2,  // alpha of iterations with parity 0 / 1 (two slots)
     SC_IT0 = SC_ALPHA_P + 2,      // first iteration of the current batch of CG iterations
     SC_TOL,                       // relative tolerance of the current solve
+    SC_ABORT,                     // nonzero: the persistent CG gave up a wait
     SC_COUNT = 32
 };
 
@@ -142,6 +143,20 @@ struct lpm_ctx {
     int cg_graph = 0;
     hipGraphExec_t cg_exec = nullptr;
     std::vector<uintptr_t> cg_key;
+    // Persistent CG (mode "cg_persist", kernels_pcg.hip): workgroups and slices per workgroup, the
+    // slots they exchange partial sums in, and each workgroup's rows by aggregate
+    int cg_persist = 1;
+    double cg_wait_ms = 2000;         // longest wait inside the kernel before the solve is done by launches
+    int pcg_state = 0, pcg_coarse = 0;  // 0 not prepared, 1 usable, -1 not; whether it has the coarse lists
+    int pcg_spw = 0, pcg_grid = 0, pcg_nslot_c = 0, pcg_nl = 0;  // pcg_nl: most aggregates of a workgroup
+    int64_t pcg_words = 0, st_pcg = 0;  // st_pcg: solves it did
+    void *pcg_slots = nullptr;
+    const void *pcg_kern = nullptr;   // the kernel and LDS size the next two were found for
+    size_t pcg_lds = 0;
+    bool pcg_fits = false;            // its whole grid can be resident
+    int pcg_khz = 0;                  // rate of the device's wall clock
+    int32_t *pcg_lptr = nullptr, *pcg_lagg = nullptr, *pcg_lslot = nullptr, *pcg_lbeg = nullptr, *pcg_wpos = nullptr,
+            *pcg_cnt = nullptr, *pcg_order = nullptr;
     int coarse_graph = 0;             // 1: replay the inversion from a HIP graph, 0: launch directly
     // Load-step predictor (mode "predictor"): free DoFs start each step from the converged
     // position extrapolated from the previous converged steps: 1 linearly (plus the previous
@@ -289,6 +304,9 @@ int coarse_check(lpm_ctx *c);  // queues the coarse-reuse mask comparison (kerne
 // diagonal; 2 adds the coarse correction
 static inline bool block_jacobi(const lpm_ctx *c) { return c->precond == 1; }
 static inline bool two_level(const lpm_ctx *c) { return c->precond == 2; }
+// ---- persistent CG (kernels_pcg.hip)
+int pcg_solve(lpm_ctx *c, int64_t maxit, bool *ran);  // the whole solve in one launch where the rule allows it
+void pcg_free(lpm_ctx *c);
 // ---- two-level preconditioner (kernels_coarse.hip)
 int coarse_prepare(lpm_ctx *c);
 int launch_coarse_apply(lpm_ctx *c);  // cz = P^T r, cy = Ac^-1 cz (skipped once the CG is done)
