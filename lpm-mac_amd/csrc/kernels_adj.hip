@@ -23,51 +23,105 @@
 
 namespace {
 
-// pass 1, one thread per particle: d dis, d cs and d f of each of its bonds
-__global__ __launch_bounds__(256) void k_jvp_bond(int64_t n, int dim, const int32_t *__restrict__ bptr,
-                                                   const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
-                                                   const double *__restrict__ dis, const double *__restrict__ cs,
-                                                   const double *__restrict__ Kn, const double *__restrict__ Tv,
-                                                   const double *__restrict__ bdamage, const double *__restrict__ v,
-                                                   double *__restrict__ dcs, double *__restrict__ dfb) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int b0 = bptr[i], bm = bsplit[i], b1 = bptr[i + 1];
-    double vi[3] = {0, 0, 0};
-    for (int k = 0; k < dim; ++k) vi[k] = v[(int64_t)dim * i + k];
-    double tot[2] = {0.0, 0.0};
-    for (int b = b0; b < b1; ++b) {
-        const int64_t j = p2[b];
-        const bool broken = fabs(bdamage[b] - 1.0) < LPM_EPS;
-        double dd[3] = {0, 0, 0};
-        for (int k = 0; k < dim; ++k) dd[k] = vi[k] - v[(int64_t)dim * j + k];
-        const double c0 = cs[3 * b], c1 = cs[3 * b + 1], c2 = cs[3 * b + 2];
-        const double ddis = broken ? 0.0 : (c0 * dd[0] + c1 * dd[1] + c2 * dd[2]);
-        const double inv = broken ? 0.0 : 1.0 / dis[b];
-        dcs[3 * b] = (dd[0] - c0 * ddis) * inv;
-        dcs[3 * b + 1] = (dd[1] - c1 * ddis) * inv;
-        dcs[3 * b + 2] = (dd[2] - c2 * ddis) * inv;
-        dfb[b] = ddis;  // d dLe for now
-        tot[b < bm ? 0 : 1] += ddis;
-    }
-    for (int b = b0; b < b1; ++b)
-        dfb[b] = (2.0 * Kn[b] * dfb[b] + 2.0 * Tv[b] * tot[b < bm ? 0 : 1]) * (1.0 - bdamage[b]);
+// The four product kernels below are bound by the per-bond arrays they read. As in the force
+// kernels, a workgroup of one wavefront owns LPM_BOND_GP consecutive particles and takes their bonds a
+// lane each, so these reads are contiguous; the per-particle sums then run over values staged in
+// LDS, in bond order. One thread per particle, each walking its own 18 bonds, took 60 + 40 us (J v) and
+// 61 + 78 us (J^T w) at SC 30 x 31 x 29.
+constexpr int GP = LPM_BOND_GP;
+
+// The particles and bonds of this workgroup; own[t] is the particle rank of bond B0 + t
+struct BondGroup {
+    int64_t p0;
+    int np, B0, nbk;
+    const int *ptr;
+};
+
+__device__ __forceinline__ BondGroup bond_group(int64_t n, const int32_t *__restrict__ bptr, int *sbp, int *own) {
+    const int tid = threadIdx.x;
+    BondGroup g;
+    g.p0 = (int64_t)blockIdx.x * GP;
+    g.np = (int)((n - g.p0) < GP ? (n - g.p0) : GP);
+    if (tid <= g.np) sbp[tid] = bptr[g.p0 + tid];
+    __syncthreads();
+    g.B0 = sbp[0];
+    g.nbk = sbp[g.np] - g.B0;
+    g.ptr = sbp;
+    // eight lanes per particle
+    const int p = tid >> 3;
+    if (p < g.np)
+        for (int b = sbp[p] + (tid & 7); b < sbp[p + 1]; b += 8) own[b - g.B0] = p;
+    __syncthreads();
+    return g;
 }
 
-// pass 2, one thread per particle: d Pin_i (dim entries per particle)
-__global__ __launch_bounds__(256) void k_jvp_particle(int64_t n, int dim, const int32_t *__restrict__ bptr,
-                                                       const int32_t *__restrict__ opp, const double *__restrict__ cs,
-                                                       const double *__restrict__ bforce, const double *__restrict__ dcs,
-                                                       const double *__restrict__ dfb, double *__restrict__ jv) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double P[3] = {0, 0, 0};
-    for (int b = bptr[i]; b < bptr[i + 1]; ++b) {
-        const int o = opp[b];
-        const double f = 0.5 * (bforce[b] + bforce[o]), df = 0.5 * (dfb[b] + dfb[o]);
-        for (int k = 0; k < 3; ++k) P[k] += dcs[3 * b + k] * f + cs[3 * b + k] * df;
+// pass 1: d f of each bond
+__global__ __launch_bounds__(64) void k_jvp_bond(int64_t n, int dim, const int32_t *__restrict__ bptr,
+                                                  const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
+                                                  const double *__restrict__ cs, const double *__restrict__ Kn,
+                                                  const double *__restrict__ Tv, const double *__restrict__ bdamage,
+                                                  const double *__restrict__ v, double *__restrict__ dfb) {
+    extern __shared__ double lds[];
+    __shared__ int sbp[GP + 1], ssp[GP];
+    __shared__ double tot[GP][2];
+    const int tid = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * GP, last = first + GP < n ? first + GP : n;
+    int *own = (int *)(lds + (bptr[last] - bptr[first]));
+    const BondGroup g = bond_group(n, bptr, sbp, own);
+    if (tid < g.np) ssp[tid] = bsplit[g.p0 + tid];
+    for (int t = tid; t < g.nbk; t += 64) {
+        const int b = g.B0 + t;
+        const int64_t i = g.p0 + own[t], j = p2[b];
+        double d = 0.0;
+        for (int k = 0; k < dim; ++k) d += cs[3 * (int64_t)b + k] * (v[dim * i + k] - v[dim * j + k]);
+        lds[t] = fabs(bdamage[b] - 1.0) < LPM_EPS ? 0.0 : d;
     }
-    for (int k = 0; k < dim; ++k) jv[(int64_t)dim * i + k] = P[k];
+    __syncthreads();
+    if (tid < 2 * g.np) {
+        const int p = tid >> 1, l = tid & 1;
+        double s = 0.0;
+        for (int t = (l ? ssp[p] : sbp[p]) - g.B0; t < (l ? sbp[p + 1] : ssp[p]) - g.B0; ++t) s += lds[t];
+        tot[p][l] = s;
+    }
+    __syncthreads();
+    for (int t = tid; t < g.nbk; t += 64) {
+        const int b = g.B0 + t, p = own[t];
+        dfb[b] = (2.0 * Kn[b] * lds[t] + 2.0 * Tv[b] * tot[p][b < ssp[p] ? 0 : 1]) * (1.0 - bdamage[b]);
+    }
+}
+
+// pass 2: d Pin_i (dim entries per particle); d cs is formed here from v again, which reads less than
+// storing it in pass 1
+__global__ __launch_bounds__(64) void k_jvp_particle(int64_t n, int dim, const int32_t *__restrict__ bptr,
+                                                      const int32_t *__restrict__ p2, const int32_t *__restrict__ opp,
+                                                      const double *__restrict__ dis, const double *__restrict__ cs,
+                                                      const double *__restrict__ bforce, const double *__restrict__ bdamage,
+                                                      const double *__restrict__ dfb, const double *__restrict__ v,
+                                                      double *__restrict__ jv) {
+    extern __shared__ double lds[];
+    __shared__ int sbp[GP + 1];
+    const int64_t first = (int64_t)blockIdx.x * GP, last = first + GP < n ? first + GP : n;
+    const int nbk = bptr[last] - bptr[first];
+    int *own = (int *)(lds + 3 * (size_t)nbk);
+    const BondGroup g = bond_group(n, bptr, sbp, own);
+    for (int t = threadIdx.x; t < nbk; t += 64) {
+        const int64_t b = g.B0 + t, i = g.p0 + own[t], j = p2[b], o = opp[b];
+        const bool broken = fabs(bdamage[b] - 1.0) < LPM_EPS;
+        double dd[3] = {0, 0, 0}, c[3];
+        for (int k = 0; k < dim; ++k) dd[k] = v[dim * i + k] - v[dim * j + k];
+        for (int k = 0; k < 3; ++k) c[k] = cs[3 * b + k];
+        const double ddis = broken ? 0.0 : (c[0] * dd[0] + c[1] * dd[1] + c[2] * dd[2]);
+        const double inv = broken ? 0.0 : 1.0 / dis[b];
+        const double f = 0.5 * (bforce[b] + bforce[o]), df = 0.5 * (dfb[b] + dfb[o]);
+        for (int k = 0; k < 3; ++k) lds[k * nbk + t] = (dd[k] - c[k] * ddis) * inv * f + c[k] * df;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < 3 * g.np) {
+        const int p = threadIdx.x / 3, k = threadIdx.x - 3 * p;
+        double s = 0.0;
+        for (int t = sbp[p] - g.B0; t < sbp[p + 1] - g.B0; ++t) s += lds[k * nbk + t];
+        if (k < dim) jv[dim * (g.p0 + p) + k] = s;
+    }
 }
 
 // Transposed product y = J^T w of the same Jacobian. J is not symmetric once the bonds of a
@@ -81,62 +135,86 @@ __global__ __launch_bounds__(256) void k_jvp_particle(int64_t n, int dim, const 
 //   a_b = (f_b + f_o) / (2 dis_b),
 //   y_i = sum over the bonds b of i of
 //         a_b (I - cs_b cs_b^T) w_i - a_o (I - cs_o cs_o^T) w_j + c_b cs_b - c_o cs_o.
-// pass 1, one thread per particle: c_b of each of its bonds
-__global__ __launch_bounds__(256) void k_vjp_bond(int64_t n, int dim, const int32_t *__restrict__ bptr,
-                                                   const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
-                                                   const int32_t *__restrict__ opp, const double *__restrict__ cs,
-                                                   const double *__restrict__ Kn, const double *__restrict__ Tv,
-                                                   const double *__restrict__ bdamage, const double *__restrict__ w,
-                                                   double *__restrict__ cb) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int b0 = bptr[i], bm = bsplit[i], b1 = bptr[i + 1];
-    double wi[3] = {0, 0, 0};
-    for (int k = 0; k < dim; ++k) wi[k] = w[(int64_t)dim * i + k];
-    double T[2] = {0.0, 0.0};
-    for (int b = b0; b < b1; ++b) {
-        const int64_t j = p2[b];
-        const int o = opp[b];
-        double t = 0.0;
-        for (int k = 0; k < dim; ++k) t += cs[3 * b + k] * wi[k] + cs[3 * (int64_t)o + k] * w[(int64_t)dim * j + k];
-        t *= 0.5;
-        cb[b] = t;  // t_b for now
-        T[b < bm ? 0 : 1] += 2.0 * Tv[b] * t * (1.0 - bdamage[b]);
+// pass 1: c_b of each bond
+__global__ __launch_bounds__(64) void k_vjp_bond(int64_t n, int dim, const int32_t *__restrict__ bptr,
+                                                  const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
+                                                  const int32_t *__restrict__ opp, const double *__restrict__ cs,
+                                                  const double *__restrict__ Kn, const double *__restrict__ Tv,
+                                                  const double *__restrict__ bdamage, const double *__restrict__ w,
+                                                  double *__restrict__ cb) {
+    extern __shared__ double lds[];
+    __shared__ int sbp[GP + 1], ssp[GP];
+    __shared__ double T[GP][2];
+    const int tid = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * GP, last = first + GP < n ? first + GP : n;
+    const int nbk = bptr[last] - bptr[first];
+    double *st = lds, *sT = lds + nbk;
+    int *own = (int *)(lds + 2 * (size_t)nbk);
+    const BondGroup g = bond_group(n, bptr, sbp, own);
+    if (tid < g.np) ssp[tid] = bsplit[g.p0 + tid];
+    for (int t = tid; t < nbk; t += 64) {
+        const int64_t b = g.B0 + t, i = g.p0 + own[t], j = p2[b], o = opp[b];
+        double x = 0.0;
+        for (int k = 0; k < dim; ++k) x += cs[3 * b + k] * w[dim * i + k] + cs[3 * o + k] * w[dim * j + k];
+        x *= 0.5;
+        st[t] = x;
+        sT[t] = 2.0 * Tv[b] * x * (1.0 - bdamage[b]);
     }
-    for (int b = b0; b < b1; ++b) {
+    __syncthreads();
+    if (tid < 2 * g.np) {
+        const int p = tid >> 1, l = tid & 1;
+        double s = 0.0;
+        for (int t = (l ? ssp[p] : sbp[p]) - g.B0; t < (l ? sbp[p + 1] : ssp[p]) - g.B0; ++t) s += sT[t];
+        T[p][l] = s;
+    }
+    __syncthreads();
+    for (int t = tid; t < nbk; t += 64) {
+        const int64_t b = g.B0 + t;
+        const int p = own[t];
         const bool broken = fabs(bdamage[b] - 1.0) < LPM_EPS;
-        cb[b] = broken ? 0.0 : 2.0 * Kn[b] * cb[b] * (1.0 - bdamage[b]) + T[b < bm ? 0 : 1];
+        cb[b] = broken ? 0.0 : 2.0 * Kn[b] * st[t] * (1.0 - bdamage[b]) + T[p][b < ssp[p] ? 0 : 1];
     }
 }
 
-// pass 2, one thread per particle: y_i
-__global__ __launch_bounds__(256) void k_vjp_particle(int64_t n, int dim, const int32_t *__restrict__ bptr,
-                                                       const int32_t *__restrict__ p2, const int32_t *__restrict__ opp,
-                                                       const double *__restrict__ dis, const double *__restrict__ cs,
-                                                       const double *__restrict__ bforce, const double *__restrict__ bdamage,
-                                                       const double *__restrict__ cb, const double *__restrict__ w,
-                                                       double *__restrict__ y) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double wi[3] = {0, 0, 0};
-    for (int k = 0; k < dim; ++k) wi[k] = w[(int64_t)dim * i + k];
-    double Y[3] = {0, 0, 0};
-    for (int b = bptr[i]; b < bptr[i + 1]; ++b) {
-        const int64_t j = p2[b];
-        const int o = opp[b];
-        double wj[3] = {0, 0, 0};
-        for (int k = 0; k < dim; ++k) wj[k] = w[(int64_t)dim * j + k];
-        const double cb_[3] = {cs[3 * b], cs[3 * b + 1], cs[3 * b + 2]};
-        const double co[3] = {cs[3 * (int64_t)o], cs[3 * (int64_t)o + 1], cs[3 * (int64_t)o + 2]};
+// pass 2: y_i
+__global__ __launch_bounds__(64) void k_vjp_particle(int64_t n, int dim, const int32_t *__restrict__ bptr,
+                                                      const int32_t *__restrict__ p2, const int32_t *__restrict__ opp,
+                                                      const double *__restrict__ dis, const double *__restrict__ cs,
+                                                      const double *__restrict__ bforce, const double *__restrict__ bdamage,
+                                                      const double *__restrict__ cb, const double *__restrict__ w,
+                                                      double *__restrict__ y) {
+    extern __shared__ double lds[];
+    __shared__ int sbp[GP + 1];
+    const int64_t first = (int64_t)blockIdx.x * GP, last = first + GP < n ? first + GP : n;
+    const int nbk = bptr[last] - bptr[first];
+    int *own = (int *)(lds + 3 * (size_t)nbk);
+    const BondGroup g = bond_group(n, bptr, sbp, own);
+    for (int t = threadIdx.x; t < nbk; t += 64) {
+        const int64_t b = g.B0 + t, i = g.p0 + own[t], j = p2[b], o = opp[b];
+        double wi[3] = {0, 0, 0}, wj[3] = {0, 0, 0}, c[3], co[3];
+        for (int k = 0; k < dim; ++k) {
+            wi[k] = w[dim * i + k];
+            wj[k] = w[dim * j + k];
+        }
+        for (int k = 0; k < 3; ++k) {
+            c[k] = cs[3 * b + k];
+            co[k] = cs[3 * o + k];
+        }
         const double f = 0.5 * (bforce[b] + bforce[o]);
         const double ab = fabs(bdamage[b] - 1.0) < LPM_EPS ? 0.0 : f / dis[b];
         const double ao = fabs(bdamage[o] - 1.0) < LPM_EPS ? 0.0 : f / dis[o];
-        const double pb = cb_[0] * wi[0] + cb_[1] * wi[1] + cb_[2] * wi[2];
+        const double pb = c[0] * wi[0] + c[1] * wi[1] + c[2] * wi[2];
         const double po = co[0] * wj[0] + co[1] * wj[1] + co[2] * wj[2];
-        for (int k = 0; k < 3; ++k)
-            Y[k] += ab * (wi[k] - cb_[k] * pb) - ao * (wj[k] - co[k] * po) + cb[b] * cb_[k] - cb[o] * co[k];
+        const double cbb = cb[b], cbo = cb[o];
+        for (int k = 0; k < 3; ++k) lds[k * nbk + t] = ab * (wi[k] - c[k] * pb) - ao * (wj[k] - co[k] * po) + cbb * c[k] - cbo * co[k];
     }
-    for (int k = 0; k < dim; ++k) y[(int64_t)dim * i + k] = Y[k];
+    __syncthreads();
+    if ((int)threadIdx.x < 3 * g.np) {
+        const int p = threadIdx.x / 3, k = threadIdx.x - 3 * p;
+        double s = 0.0;
+        for (int t = sbp[p] - g.B0; t < sbp[p + 1] - g.B0; ++t) s += lds[k * nbk + t];
+        if (k < dim) y[dim * (g.p0 + p) + k] = s;
+    }
 }
 
 // Zero the entries of DoFs that the Dirichlet elimination removes (constrained, or of a fully
@@ -554,27 +632,27 @@ static int check(lpm_ctx *c, const char *what) {
     return LPM_OK;
 }
 
-// the context's per-bond scratch (4 doubles per bond; kernels on the context stream use it in
+// the context's per-bond scratch (one double per bond; kernels on the context stream use it in
 // turn, so one buffer serves every product)
 static int adj_scratch(lpm_ctx *c, double **p) {
-    if (!c->adj_scr) LPM_HIP(c, hipMalloc(&c->adj_scr, sizeof(double) * 4 * std::max<int64_t>(c->nbond, 1)));
+    if (!c->adj_scr) LPM_HIP(c, hipMalloc(&c->adj_scr, sizeof(double) * std::max<int64_t>(c->nbond, 1)));
     *p = c->adj_scr;
     return LPM_OK;
 }
 
 // jv = dPin/dx . v at the current geometry and forces (both dim*n, device)
 int force_jvp(lpm_ctx *c, const double *v, double *jv) {
-    const int g = blocks_for(c->n, 256);
-    double *dcs = nullptr;
-    int rc = adj_scratch(c, &dcs);
+    const int g = blocks_for(c->n, GP);
+    double *dfb = nullptr;
+    int rc = adj_scratch(c, &dfb);
     if (rc) return rc;
-    double *dfb = dcs + 3 * std::max<int64_t>(c->nbond, 1);
-    hipLaunchKernelGGL(k_jvp_bond, dim3(g), dim3(256), 0, c->stream, c->n, c->dim, c->bptr, c->bsplit, c->p2, c->dis, c->cs,
-                       c->Kn, c->Tv, c->bdamage, v, dcs, dfb);
+    const size_t nb = c->gp_bonds;  // most bonds of a workgroup's particles
+    hipLaunchKernelGGL(k_jvp_bond, dim3(g), dim3(64), nb * (sizeof(double) + sizeof(int)), c->stream, c->n, c->dim, c->bptr,
+                       c->bsplit, c->p2, c->cs, c->Kn, c->Tv, c->bdamage, v, dfb);
     rc = check(c, "k_jvp_bond");
     if (!rc) {
-        hipLaunchKernelGGL(k_jvp_particle, dim3(g), dim3(256), 0, c->stream, c->n, c->dim, c->bptr, c->opp, c->cs, c->bforce,
-                           dcs, dfb, jv);
+        hipLaunchKernelGGL(k_jvp_particle, dim3(g), dim3(64), nb * (3 * sizeof(double) + sizeof(int)), c->stream, c->n, c->dim,
+                           c->bptr, c->p2, c->opp, c->dis, c->cs, c->bforce, c->bdamage, dfb, v, jv);
         rc = check(c, "k_jvp_particle");
     }
     return rc;
@@ -582,16 +660,17 @@ int force_jvp(lpm_ctx *c, const double *v, double *jv) {
 
 // y = (dPin/dx)^T w at the current geometry and forces (both dim*n, device)
 int force_vjp(lpm_ctx *c, const double *w, double *y) {
-    const int g = blocks_for(c->n, 256);
+    const int g = blocks_for(c->n, GP);
     double *cb = nullptr;
     int rc = adj_scratch(c, &cb);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_vjp_bond, dim3(g), dim3(256), 0, c->stream, c->n, c->dim, c->bptr, c->bsplit, c->p2, c->opp, c->cs,
-                       c->Kn, c->Tv, c->bdamage, w, cb);
+    const size_t nb = c->gp_bonds;
+    hipLaunchKernelGGL(k_vjp_bond, dim3(g), dim3(64), nb * (2 * sizeof(double) + sizeof(int)), c->stream, c->n, c->dim, c->bptr,
+                       c->bsplit, c->p2, c->opp, c->cs, c->Kn, c->Tv, c->bdamage, w, cb);
     rc = check(c, "k_vjp_bond");
     if (!rc) {
-        hipLaunchKernelGGL(k_vjp_particle, dim3(g), dim3(256), 0, c->stream, c->n, c->dim, c->bptr, c->p2, c->opp, c->dis, c->cs,
-                           c->bforce, c->bdamage, cb, w, y);
+        hipLaunchKernelGGL(k_vjp_particle, dim3(g), dim3(64), nb * (3 * sizeof(double) + sizeof(int)), c->stream, c->n, c->dim,
+                           c->bptr, c->p2, c->opp, c->dis, c->cs, c->bforce, c->bdamage, cb, w, y);
         rc = check(c, "k_vjp_particle");
     }
     return rc;

@@ -186,7 +186,7 @@ struct lpm_ctx {
     // state a converged step leaves (positions, loads, constraint flags, particle and bond state
     // and their last-converged copies); null where the slot is empty
     std::vector<void *> ckpt;
-    // per-bond scratch of the force JVP / VJP (4 doubles per bond), allocated on first use
+    // per-bond scratch of the force JVP / VJP (a double per bond), allocated on first use
     double *adj_scr = nullptr;
     // the last fatigue damage update (SolverFatigue::updateFatigueDamage): positions its nonlocal
     // weights used and each particle's energy range s2 - s1 (the update resets both), its cycle
