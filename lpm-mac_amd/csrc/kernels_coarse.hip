@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void k_coarse_blocks(int64_t ncq, const int32_
 }
 
 // Blocked Gauss-Jordan inversion of the symmetrised Ac (SPD, so no pivoting), NB pivots per
-// block step, two launches per step (reading A_in, writing A_out, so no element is read after
+// block step, one launch per step (reading A_in, writing A_out, so no element is read after
 // another thread wrote it). A coarse DoF whose row is zero (an aggregate whose DoFs are all
 // eliminated) is set to the identity before and to zero after, so it receives no correction.
 // A coarse DoF whose pivot (its Schur complement against the pivots before it) falls to
@@ -168,85 +168,87 @@ __global__ __launch_bounds__(256) void k_coarse_dead(int ncoarse, int M, const i
     }
 }
 
-// Block step kb, part 1 (one workgroup per group): Dinv = A[K,K]^-1 by Gauss-Jordan in LDS, with
-// the pivot drop described above. Dinv is stored NB x NB (row stride NB), zero outside nb x nb
-// and in the rows and columns of dropped pivots.
-__global__ __launch_bounds__(1024) void k_gj_diag(int kb, const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
-                                                   const double *__restrict__ Ain, const double *__restrict__ odiag_all,
-                                                   uint8_t *__restrict__ dead_all, double *__restrict__ Dinv_all) {
-    __shared__ double D[GJ_NB][GJ_NB + 1];
-    __shared__ uint8_t skip[GJ_NB];
-    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
-    if (kb >= nc) return;  // this group's inversion has finished
-    const double *A = Ain + off[b];
-    const int nb = min(GJ_NB, nc - kb);
-    const int tid = threadIdx.x, i = tid / GJ_NB, j = tid % GJ_NB;  // blockDim = NB * NB
-    const bool in = i < nb && j < nb;
-    D[i][j] = in ? A[(int64_t)(kb + i) * nc + kb + j] : 0.0;
-    if (tid < GJ_NB) skip[tid] = 0;
-    __syncthreads();
-    for (int k = 0; k < nb; ++k) {
-        // every thread reads the same pivot, so the skip branch is uniform across the workgroup
-        const double pk = D[k][k];
-        if (!(pk > GJ_DROP * odiag_all[base + kb + k])) {
-            if (tid == 0) {
-                skip[k] = 1;
-                dead_all[base + kb + k] = 1;
-            }
+// Dinv = A[K,K]^-1 of the nb x nb pivot block in D by Gauss-Jordan with the pivot drop described
+// above, by one wavefront: lane (h, i) holds columns 16h .. 16h+15 of row i in registers, and each pivot's row
+// and column pass through LDS without a barrier. 32 pivots take 5 us; a workgroup of one
+// thread per element with two barriers per pivot took 16 us. Dinv is NB x NB, zero outside nb x nb and in the rows and
+// columns of dropped pivots.
+__device__ __forceinline__ void gj_invert(const double (&D)[GJ_NB][GJ_NB + 1], double (*rc)[GJ_NB], int nb, const double *odiag,
+                                          uint8_t *dead, double *Dinv) {
+    const int lane = threadIdx.x & 63, h = lane >> 5, i = lane & 31;
+    double d[16];
+    unsigned skip = 0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) d[q] = D[i][16 * h + q];
+#pragma unroll
+    for (int k = 0; k < GJ_NB; ++k) {
+        if (k >= nb) break;
+        // the pivot row (all columns) and column (all rows) to every lane
+        if (i == k)
+            for (int q = 0; q < 16; ++q) rc[0][16 * h + q] = d[q];
+        if (h == (k >> 4)) rc[1][i] = d[k & 15];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const double pk = rc[0][k], ck = rc[1][i];
+        double r[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) r[q] = rc[0][16 * h + q];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (!(pk > GJ_DROP * odiag[k])) {  // the same for every lane
+            skip |= 1u << k;
+            if (lane == 0) dead[k] = 1;
             continue;
         }
-        const double rk = (j == k) ? 1.0 : D[k][j], ck = D[i][k];
-        __syncthreads();
-        if (in) {
-            const double p = 1.0 / pk;
-            if (i == k) D[i][j] = rk * p;
-            else D[i][j] = ((j == k) ? 0.0 : D[i][j]) - ck * rk * p;
+        const double p = 1.0 / pk;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const bool piv = 16 * h + q == k;
+            const double rk = piv ? 1.0 : r[q];
+            if (i == k) d[q] = rk * p;
+            else d[q] = (piv ? 0.0 : d[q]) - ck * rk * p;
         }
-        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int j = 16 * h + q;
+        Dinv[i * GJ_NB + j] = (i < nb && j < nb && !((skip >> i) & 1) && !((skip >> j) & 1)) ? d[q] : 0.0;
+    }
+}
+
+// The first pivot block of every group
+__global__ __launch_bounds__(64) void k_gj_diag(const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
+                                                const double *__restrict__ Ain, const double *__restrict__ odiag_all,
+                                                uint8_t *__restrict__ dead_all, double *__restrict__ Dinv_all) {
+    __shared__ double D[GJ_NB][GJ_NB + 1], rc[2][GJ_NB];
+    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
+    if (nc <= 0) return;
+    const double *A = Ain + off[b];
+    const int nb = min(GJ_NB, nc);
+    for (int e = threadIdx.x; e < GJ_NB * GJ_NB; e += 64) {
+        const int i = e / GJ_NB, j = e % GJ_NB;
+        D[i][j] = i < nb && j < nb ? A[(int64_t)i * nc + j] : 0.0;
     }
     __syncthreads();
-    Dinv_all[(int64_t)b * GJ_NB * GJ_NB + tid] = (in && !skip[i] && !skip[j]) ? D[i][j] : 0.0;
+    gj_invert(D, rc, nb, odiag_all + base, dead_all + base, Dinv_all + (int64_t)b * GJ_NB * GJ_NB);
 }
 
-// Block step kb, part 2: the row panel Rt[j][k] = sum_m Dinv[k][m] A[kb+m][j] for j outside K
-// (zero for j in K), row stride NB; four threads per column j, eight k each, Dinv staged in LDS.
-__global__ __launch_bounds__(256) void k_gj_panel(int kb, const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
-                                                   const double *__restrict__ Ain, const double *__restrict__ Dinv_all,
-                                                   double *__restrict__ Rt_all) {
-    __shared__ double Ds[GJ_NB][GJ_NB + 1];
-    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
-    if (kb >= nc || (int)(blockIdx.x * (blockDim.x >> 2)) >= nc) return;  // uniform over the workgroup
-    const double *Dinv = Dinv_all + (int64_t)b * GJ_NB * GJ_NB;
-    for (int e = threadIdx.x; e < GJ_NB * GJ_NB; e += blockDim.x) Ds[e / GJ_NB][e % GJ_NB] = Dinv[e];
-    __syncthreads();
-    const int t = blockIdx.x * blockDim.x + threadIdx.x, j = t >> 2, k0 = (t & 3) * 8;
-    if (j >= nc) return;
-    const double *A = Ain + off[b];
-    const int nb = min(GJ_NB, nc - kb);
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (j < kb || j >= kb + nb)
-        for (int m = 0; m < nb; ++m) {
-            const double a = A[(int64_t)(kb + m) * nc + j];
-            for (int q = 0; q < 8; ++q) acc[q] += Ds[k0 + q][m] * a;
-        }
-    double *Rt = Rt_all + (int64_t)(base + j) * GJ_NB + k0;
-    for (int q = 0; q < 8; ++q) Rt[q] = acc[q];
-}
-
-// Block step kb, part 3: the rank-NB update of the group's block, one 32 x 32 tile per
-// workgroup (tiles are aligned with the pivot blocks, so a tile lies wholly inside or outside K
-// in each direction):
+// Block step kb: the rank-NB update of the group's block, one 32 x 32 tile per workgroup (tiles are
+// aligned with the pivot blocks, so a tile lies wholly inside or outside K in each direction). With
+// R = Dinv A[K, :]:
 //   tile in K x K:      Dinv
-//   row tile in K:      Rt^T
+//   row tile in K:      R
 //   column tile in K:   -A[:,K] Dinv
-//   else:               A - A[:,K] Rt^T
-// A group whose inversion has finished is copied, so that every block ends in the same buffer.
-__global__ __launch_bounds__(256) void k_gj_update(int kb, int T, const int32_t *__restrict__ cb,
-                                                    const int64_t *__restrict__ off, const double *__restrict__ Ain_all,
-                                                    double *__restrict__ Aout_all, const double *__restrict__ Dinv_all,
-                                                    const double *__restrict__ Rt_all) {
+//   else:               A - A[:,K] R
+// Each workgroup forms its own 32 columns of R, and the one whose tile is the next pivot block inverts it
+// for the next step (into the other Dinv), so a step is one launch instead of three (inversion
+// 15.6, panel 7.0, update 12.8 us). A group whose inversion has finished is copied, so that every block ends in the same buffer.
+__global__ __launch_bounds__(256) void k_gj_step(int kb, int T, const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
+                                                  const double *__restrict__ Ain_all, double *__restrict__ Aout_all,
+                                                  const double *__restrict__ Dinv_all, double *__restrict__ Dnext_all,
+                                                  const double *__restrict__ odiag_all, uint8_t *__restrict__ dead_all) {
     static_assert(GJ_NB == 32, "tiles are 32 x 32 pivot blocks");
-    __shared__ double L[32][33], R[32][33];
+    __shared__ double L[32][33], R[32][33], X[32][33], rc[2][32];
     const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
     const int i0 = (blockIdx.x / T) * 32, j0 = (blockIdx.x % T) * 32;
     if (i0 >= nc || j0 >= nc) return;  // uniform over the workgroup
@@ -260,35 +262,47 @@ __global__ __launch_bounds__(256) void k_gj_update(int kb, int T, const int32_t 
         }
         return;
     }
-    const double *Dinv = Dinv_all + (int64_t)b * GJ_NB * GJ_NB, *Rt = Rt_all + (int64_t)base * GJ_NB;
+    const double *Dinv = Dinv_all + (int64_t)b * GJ_NB * GJ_NB;
     const int nb = min(GJ_NB, nc - kb);
     const bool ik = i0 == kb, jk = j0 == kb;
-    if (ik && jk) {
-        for (int q = 0; q < 4; ++q) {
-            const int ii = ty + 8 * q, i = i0 + ii, j = j0 + tx;
-            if (i < nc && j < nc) Aout[(int64_t)i * nc + j] = Dinv[ii * GJ_NB + tx];
-        }
-        return;
-    }
-    for (int e = threadIdx.x; e < 32 * 32; e += blockDim.x) {
-        const int r = e >> 5, m = e & 31;
-        // R[jj][m]: Rt rows j0.. (row tile in K and general case) or Dinv^T (column tile in K)
-        R[r][m] = jk ? Dinv[m * GJ_NB + r] : ((j0 + r < nc) ? Rt[(int64_t)(j0 + r) * GJ_NB + m] : 0.0);
-        L[r][m] = (!ik && i0 + r < nc && m < nb) ? Ain[(int64_t)(i0 + r) * nc + kb + m] : 0.0;
+    // X = Dinv; L = A[i0.., K]; R = A[K, j0..] (the tile of Dinv itself where j0 is in K)
+    double a[4];
+    for (int q = 0; q < 4; ++q) {
+        const int r = ty + 8 * q;
+        X[r][tx] = Dinv[r * GJ_NB + tx];
+        L[r][tx] = (!ik && i0 + r < nc && tx < nb) ? Ain[(int64_t)(i0 + r) * nc + kb + tx] : 0.0;
+        R[r][tx] = (!jk && r < nb && j0 + tx < nc) ? Ain[(int64_t)(kb + r) * nc + j0 + tx] : 0.0;
+        a[q] = (!ik && !jk && i0 + r < nc && j0 + tx < nc) ? Ain[(int64_t)(i0 + r) * nc + j0 + tx] : 0.0;
     }
     __syncthreads();
+    double v[4] = {0, 0, 0, 0};
+    if (jk) {
+        for (int q = 0; q < 4; ++q) v[q] = X[ty + 8 * q][tx];
+    } else {
+        for (int m = 0; m < 32; ++m)
+            for (int q = 0; q < 4; ++q) v[q] += X[ty + 8 * q][m] * R[m][tx];
+    }
+    if (!ik) {
+        __syncthreads();
+        for (int q = 0; q < 4; ++q) R[ty + 8 * q][tx] = v[q];  // R = Dinv A[K, j0..], or Dinv
+        __syncthreads();
+        double t[4] = {0, 0, 0, 0};
+        for (int m = 0; m < 32; ++m)
+            for (int q = 0; q < 4; ++q) t[q] += L[ty + 8 * q][m] * R[m][tx];
+        for (int q = 0; q < 4; ++q) v[q] = jk ? -t[q] : a[q] - t[q];
+    }
     for (int q = 0; q < 4; ++q) {
-        const int ii = ty + 8 * q, i = i0 + ii, j = j0 + tx;
-        if (i >= nc || j >= nc) continue;
-        double v;
-        if (ik) {
-            v = R[tx][ii];
-        } else {
-            double s = 0.0;
-            for (int m = 0; m < 32; ++m) s += L[ii][m] * R[tx][m];
-            v = jk ? -s : Ain[(int64_t)i * nc + j] - s;
-        }
-        Aout[(int64_t)i * nc + j] = v;
+        const int i = i0 + ty + 8 * q, j = j0 + tx;
+        if (i < nc && j < nc) Aout[(int64_t)i * nc + j] = v[q];
+    }
+    // the next pivot block
+    if (i0 == kb + GJ_NB && j0 == i0) {
+        __syncthreads();
+        for (int q = 0; q < 4; ++q) L[ty + 8 * q][tx] = i0 + ty + 8 * q < nc && j0 + tx < nc ? v[q] : 0.0;
+        __syncthreads();
+        if (threadIdx.x < 64)
+            gj_invert(L, rc, min(GJ_NB, nc - i0), odiag_all + base + i0, dead_all + base + i0,
+                      Dnext_all + (int64_t)b * GJ_NB * GJ_NB);
     }
 }
 
@@ -629,13 +643,12 @@ static int coarse_setup(lpm_ctx *c) {
     LPM_HIP(c, hipMalloc(&c->ra_ptr, sizeof(int32_t) * (n + 1)));
     LPM_HIP(c, hipMalloc(&c->ra_id, sizeof(int32_t) * std::max<size_t>(rid.size(), 1)));
     LPM_HIP(c, hipMalloc(&c->cvbuf, sizeof(double) * M * M * std::max<size_t>(rid.size(), 1)));
-    // two ping-pong buffers of the packed blocks, the groups' NB x NB block inverses, their row
-    // panels, the original diagonal and the dead-row flags
+    // two ping-pong buffers of the packed blocks, two sets of the groups' NB x NB block inverses, the
+    // original diagonal and the dead-row flags
     c->ncgrp = (int)nsp;
     c->cgrp_nbmax = nbmax;
     c->ac_elems = off[nsp];
-    LPM_HIP(c, hipMalloc(&c->Ac, sizeof(double) * (2 * (size_t)c->ac_elems + (size_t)nsp * GJ_NB * GJ_NB +
-                                                   (size_t)nc * GJ_NB + nc) + nc));
+    LPM_HIP(c, hipMalloc(&c->Ac, sizeof(double) * (2 * (size_t)c->ac_elems + 2 * (size_t)nsp * GJ_NB * GJ_NB + nc) + nc));
     LPM_HIP(c, hipMalloc(&c->cgrp_cb, sizeof(int32_t) * (nsp + 1)));
     LPM_HIP(c, hipMalloc(&c->cgrp_off, sizeof(int64_t) * (nsp + 1)));
     LPM_HIP(c, hipMalloc(&c->agg_grp, sizeof(int32_t) * std::max(nagg, 1)));
@@ -733,8 +746,9 @@ int coarse_prepare(lpm_ctx *c) {
                                c->cvbuf, c->agg_grp, c->cgrp_cb, c->cgrp_off, c->Ac);
         if ((rc = ck(c, "k_coarse_blocks"))) return rc;
     }
-    double *A0 = c->Ac, *A1 = c->Ac + ne, *Dinv = c->Ac + 2 * ne, *Rt = Dinv + (int64_t)G * GJ_NB * GJ_NB;
-    double *odiag = Rt + (int64_t)nc * GJ_NB;
+    const int64_t nd = (int64_t)G * GJ_NB * GJ_NB;
+    double *A0 = c->Ac, *A1 = c->Ac + ne, *Dinv = c->Ac + 2 * ne;  // two sets of block inverses
+    double *odiag = Dinv + 2 * nd;
     uint8_t *dead = (uint8_t *)(odiag + nc);
     const int nsteps = (nbmax + GJ_NB - 1) / GJ_NB, T = nsteps;  // T x T tiles of 32 cover the largest block
     // every group's block in the same launches (grid y = group, x over the largest block)
@@ -745,18 +759,14 @@ int coarse_prepare(lpm_ctx *c) {
         hipLaunchKernelGGL(k_coarse_dead, dim3(blocks_for(nc, 4)), dim3(256), 0, c->stream, nc, M,
                            (const int32_t *)c->agg_grp, (const int32_t *)c->cgrp_cb, (const int64_t *)c->cgrp_off, A0, odiag,
                            dead);
+        hipLaunchKernelGGL(k_gj_diag, dim3(1, G), dim3(64), 0, c->stream, (const int32_t *)c->cgrp_cb,
+                           (const int64_t *)c->cgrp_off, (const double *)A0, (const double *)odiag, dead, Dinv);
         for (int st = 0; st < nsteps; ++st) {
             const double *Ain = (st & 1) ? A1 : A0;
             double *Aout = (st & 1) ? A0 : A1;
-            hipLaunchKernelGGL(k_gj_diag, dim3(1, G), dim3(GJ_NB * GJ_NB), 0, c->stream, st * GJ_NB,
-                               (const int32_t *)c->cgrp_cb, (const int64_t *)c->cgrp_off, Ain, (const double *)odiag, dead,
-                               Dinv);
-            hipLaunchKernelGGL(k_gj_panel, dim3(blocks_for((int64_t)nbmax * 4, 256), G), dim3(256), 0, c->stream,
-                               st * GJ_NB, (const int32_t *)c->cgrp_cb, (const int64_t *)c->cgrp_off, Ain,
-                               (const double *)Dinv, Rt);
-            hipLaunchKernelGGL(k_gj_update, dim3(T * T, G), dim3(256), 0, c->stream, st * GJ_NB, T,
-                               (const int32_t *)c->cgrp_cb, (const int64_t *)c->cgrp_off, Ain, Aout, (const double *)Dinv,
-                               (const double *)Rt);
+            hipLaunchKernelGGL(k_gj_step, dim3(T * T, G), dim3(256), 0, c->stream, st * GJ_NB, T, (const int32_t *)c->cgrp_cb,
+                               (const int64_t *)c->cgrp_off, Ain, Aout, (const double *)(Dinv + (st & 1) * nd),
+                               Dinv + ((st + 1) & 1) * nd, (const double *)odiag, dead);
         }
         hipLaunchKernelGGL(k_coarse_undead, gsq, dim3(256), 0, c->stream, (const int32_t *)c->cgrp_cb,
                            (const int64_t *)c->cgrp_off, (nsteps & 1) ? A1 : A0, (const uint8_t *)dead);
