@@ -38,33 +38,41 @@ __global__ __launch_bounds__(256) void k_dofmask(int64_t n, int dim, const int32
     mask[i] = (uint8_t)m;
 }
 
-// Stage 1, one thread per row i: for each aggregate h among the columns of row i (in the
-// row's aggregate list), V = P_i^T (sum over slots with agg(j) = h, in slot order, of K_ij P_j).
-// With P_j = [I | R(d_j)], K_ij P_j = [K_ij | K_ij R(d_j)]. Column indices come from the SELL
-// copy (scol: slot c of row i at sp[i/64] + 64 c + i%64), which the lanes of a wavefront (the
-// 64 rows of a slice) read coalesced, where the CSR list would put every lane on its own line.
+// Stage 1, one thread per entry f = (row i, aggregate h among its columns): V = P_i^T (sum over slots
+// with agg(j) = h, in slot order, of K_ij P_j). With P_j = [I | R(d_j)], K_ij P_j = [K_ij | K_ij R(d_j)].
+// Column indices come from the SELL copy (scol: slot c of row i at sp[i/64] + 64 c + i%64); the entries of
+// neighbouring rows are neighbouring threads, so the lanes read few lines, where the CSR list would put
+// every lane on its own. A chain of dependent loads per slot bounds it (column, its aggregate, the
+// block), so what counts is threads in flight: one thread per row, taking its entries in turn, took 218
+// us at BCC 21 x 20 x 19 in FP64 (67 workgroups) and 57 us at SC 12^3.
 template <typename T, int D>
-__global__ __launch_bounds__(256) void k_coarse_rows(int64_t n, const int32_t *__restrict__ cptr,
-                                                      const int32_t *__restrict__ scol, const int64_t *__restrict__ sp,
-                                                      const T *__restrict__ aval, const int32_t *__restrict__ agg_of,
-                                                      const double *__restrict__ agg_d, const uint8_t *__restrict__ mask,
-                                                      const int32_t *__restrict__ ra_ptr, const int32_t *__restrict__ ra_id,
-                                                      double *__restrict__ vbuf) {
-    constexpr int EB = D * D, M = D == 3 ? 6 : 3;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int nc = cptr[i + 1] - cptr[i];
+__global__ __launch_bounds__(64) void k_coarse_rows(int64_t nra, const int32_t *__restrict__ cptr,
+                                                     const int32_t *__restrict__ scol, const int64_t *__restrict__ sp,
+                                                     const T *__restrict__ aval, const int32_t *__restrict__ agg_of,
+                                                     const double *__restrict__ agg_d, const uint8_t *__restrict__ mask,
+                                                     const int32_t *__restrict__ ra_row, const int32_t *__restrict__ ra_id,
+                                                     double *__restrict__ vbuf) {
+    constexpr int EB = D * D, M = D == 3 ? 6 : 3, UNR = 8;
+    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= nra) return;
+    const int64_t i = ra_row[f];
+    const int nc = cptr[i + 1] - cptr[i], h = ra_id[f];
     const int32_t *ci = scol + sp[i >> 6] + (i & 63);
-    double Pi[3][6];
-    rigid_modes<D>(&agg_d[D * i], mask[i], Pi);
-    for (int f = ra_ptr[i]; f < ra_ptr[i + 1]; ++f) {
-        const int h = ra_id[f];
-        double W[D][M];
-        for (int r = 0; r < D; ++r)
-            for (int m = 0; m < M; ++m) W[r][m] = 0.0;
-        for (int c = 0; c < nc; ++c) {
-            const int64_t j = ci[(int64_t)c * 64];
-            if (agg_of[j] != h) continue;
+    double W[D][M];
+    for (int r = 0; r < D; ++r)
+        for (int m = 0; m < M; ++m) W[r][m] = 0.0;
+    for (int c0 = 0; c0 < nc; c0 += UNR) {
+        // the columns and aggregates of several slots are requested before they are looked at
+        int32_t jc[UNR], ja[UNR];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) jc[u] = c0 + u < nc ? ci[(int64_t)(c0 + u) * 64] : -1;
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) ja[u] = jc[u] >= 0 ? agg_of[jc[u]] : -1;
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) {
+            if (ja[u] != h) continue;
+            const int64_t j = jc[u];
+            const int c = c0 + u;
             double Pj[3][6];
             rigid_modes<D>(&agg_d[D * j], mask[j], Pj);
             double Kb[D][D];
@@ -77,14 +85,16 @@ __global__ __launch_bounds__(256) void k_coarse_rows(int64_t n, const int32_t *_
                     W[r][m] += t;
                 }
         }
-        double *out = vbuf + (int64_t)f * M * M;
-        for (int a = 0; a < M; ++a)
-            for (int b = 0; b < M; ++b) {
-                double t = 0.0;
-                for (int r = 0; r < D; ++r) t += Pi[r][a] * W[r][b];
-                out[a * M + b] = t;
-            }
     }
+    double Pi[3][6];
+    rigid_modes<D>(&agg_d[D * i], mask[i], Pi);
+    double *out = vbuf + f * M * M;
+    for (int a = 0; a < M; ++a)
+        for (int b = 0; b < M; ++b) {
+            double t = 0.0;
+            for (int r = 0; r < D; ++r) t += Pi[r][a] * W[r][b];
+            out[a * M + b] = t;
+        }
 }
 
 // Stage 2, one wavefront per coarse block q = (g, h): lanes take the block's row entries in a
@@ -445,7 +455,7 @@ static int ck(lpm_ctx *c, const char *what) {
 
 void coarse_free(lpm_ctx *c) {
     if (c->gj_graph) hipGraphExecDestroy(c->gj_graph);
-    void *ptrs[] = {c->agg_of, c->agg_ptr, c->agg_idx, c->agg_d, c->ra_ptr, c->ra_id,  c->cq_ptr,
+    void *ptrs[] = {c->agg_of, c->agg_ptr, c->agg_idx, c->agg_d, c->ra_row, c->ra_id,  c->cq_ptr,
                     c->cq_f,   c->cq_gh,   c->cvbuf,   c->Ac,    c->cz,     c->cy,     c->dofmask,
                     c->cgrp_cb, c->cgrp_off, c->agg_grp, c->dofmask_prev, c->agg_dm};
     for (void *p : ptrs)
@@ -588,8 +598,9 @@ static int coarse_setup(lpm_ctx *c) {
     for (int64_t i = 0; i < n; ++i)
         for (int k = 0; k < 3; ++k) d[3 * i + k] = x[3 * i + k] - cen[3 * agg[i] + k];
     // distinct aggregates of each row's columns (ascending)
-    std::vector<int32_t> rptr(n + 1, 0), rid;
+    std::vector<int32_t> rptr(n + 1, 0), rid, rrow;
     rid.reserve(2 * n);
+    rrow.reserve(2 * n);
     for (int64_t i = 0; i < n; ++i) {
         std::vector<int32_t> hs;
         for (int q = cp[i]; q < cp[i + 1]; ++q) hs.push_back(agg[ci[q]]);
@@ -597,6 +608,7 @@ static int coarse_setup(lpm_ctx *c) {
         hs.erase(std::unique(hs.begin(), hs.end()), hs.end());
         rid.insert(rid.end(), hs.begin(), hs.end());
         rptr[i + 1] = (int32_t)rid.size();
+        rrow.resize(rid.size(), (int32_t)i);
     }
     // coarse blocks (g, h) and their contributing row entries f, in row order
     std::vector<int32_t> qgh;
@@ -640,7 +652,7 @@ static int coarse_setup(lpm_ctx *c) {
     LPM_HIP(c, hipMalloc(&c->agg_ptr, sizeof(int32_t) * (nagg + 1)));
     LPM_HIP(c, hipMalloc(&c->agg_idx, sizeof(int32_t) * n));
     LPM_HIP(c, hipMalloc(&c->agg_d, sizeof(double) * D * std::max<int64_t>(n, 1)));
-    LPM_HIP(c, hipMalloc(&c->ra_ptr, sizeof(int32_t) * (n + 1)));
+    LPM_HIP(c, hipMalloc(&c->ra_row, sizeof(int32_t) * std::max<size_t>(rid.size(), 1)));
     LPM_HIP(c, hipMalloc(&c->ra_id, sizeof(int32_t) * std::max<size_t>(rid.size(), 1)));
     LPM_HIP(c, hipMalloc(&c->cvbuf, sizeof(double) * M * M * std::max<size_t>(rid.size(), 1)));
     // two ping-pong buffers of the packed blocks, two sets of the groups' NB x NB block inverses, the
@@ -674,7 +686,7 @@ static int coarse_setup(lpm_ctx *c) {
     LPM_HIP(c, hipMemcpyAsync(c->agg_ptr, aptr.data(), sizeof(int32_t) * (nagg + 1), hipMemcpyHostToDevice, c->stream));
     LPM_HIP(c, hipMemcpyAsync(c->agg_idx, aidx.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, c->stream));
     LPM_HIP(c, hipMemcpyAsync(c->agg_d, dD.data(), sizeof(double) * D * n, hipMemcpyHostToDevice, c->stream));
-    LPM_HIP(c, hipMemcpyAsync(c->ra_ptr, rptr.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice, c->stream));
+    LPM_HIP(c, hipMemcpyAsync(c->ra_row, rrow.data(), sizeof(int32_t) * rrow.size(), hipMemcpyHostToDevice, c->stream));
     LPM_HIP(c, hipMemcpyAsync(c->ra_id, rid.data(), sizeof(int32_t) * rid.size(), hipMemcpyHostToDevice, c->stream));
     LPM_HIP(c, hipStreamSynchronize(c->stream));
     return LPM_OK;
@@ -682,8 +694,8 @@ static int coarse_setup(lpm_ctx *c) {
 
 template <typename T, int D>
 static int coarse_rows_t(lpm_ctx *c) {
-    hipLaunchKernelGGL((k_coarse_rows<T, D>), dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->cptr,
-                       c->scol, c->sp, (const T *)c->aval, c->agg_of, c->agg_d, c->dofmask, c->ra_ptr, c->ra_id, c->cvbuf);
+    hipLaunchKernelGGL((k_coarse_rows<T, D>), dim3(blocks_for(c->nra, 64)), dim3(64), 0, c->stream, c->nra, c->cptr,
+                       c->scol, c->sp, (const T *)c->aval, c->agg_of, c->agg_d, c->dofmask, c->ra_row, c->ra_id, c->cvbuf);
     return ck(c, "k_coarse_rows");
 }
 
