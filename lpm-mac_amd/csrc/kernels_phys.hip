@@ -35,8 +35,9 @@ __device__ __forceinline__ double dmin(double a, double b) { return (b < a) ? b 
 // particle_j2plasticity.h:63-76, particle_fatigue_hcf.h:65-80).
 // A workgroup of one wavefront owns GP consecutive particles and their contiguous bond range.
 // Per-bond work runs lane-per-bond (coalesced loads and stores of the bond arrays); the
-// per-particle sums then run thread-per-particle over the bond values staged in LDS, in bond
-// order, so every sum is formed in the reference's order.
+// per-particle sums then run a thread per (particle, sum) over the bond values staged in LDS, in
+// bond order, so every sum is formed in the reference's order. A thread per particle for all its
+// sums left 56 of 64 lanes idle in a serial chain: at FCC 20^3 (32k particles) 15.4 -> 14.3 us here.
 constexpr int GP = LPM_BOND_GP;  // particles per workgroup of the bond kernels
 
 __global__ __launch_bounds__(64) void k_geometry_force(
@@ -59,8 +60,8 @@ __global__ __launch_bounds__(64) void k_geometry_force(
     const int B0 = sbp[0], nbk = sbp[np] - B0;
     double *sle = lds, *stle = sle + nbk, *scx = stle + nbk, *scy = scx + nbk, *scz = scy + nbk;
     int *own = (int *)(scz + nbk);
-    if (tid < np)
-        for (int b = sbp[tid]; b < sbp[tid + 1]; ++b) own[b - B0] = tid;
+    if ((tid >> 3) < np)  // eight lanes per particle
+        for (int b = sbp[tid >> 3] + (tid & 7); b < sbp[(tid >> 3) + 1]; b += 8) own[b - B0] = tid >> 3;
     __syncthreads();
     for (int t = tid; t < nbk; t += blockDim.x) {
         const int b = B0 + t;
@@ -87,24 +88,20 @@ __global__ __launch_bounds__(64) void k_geometry_force(
         scz[t] = cz;
     }
     __syncthreads();
-    if (tid < np) {
-        const int64_t i = p0 + tid;
-        for (int l = 0; l < 2; ++l) {
-            const int lo = (l == 0 ? sbp[tid] : ssp[tid]) - B0, hi = (l == 0 ? ssp[tid] : sbp[tid + 1]) - B0;
-            double dt = 0, tdt = 0, sx = 0, sy = 0, sz = 0;
-            for (int t = lo; t < hi; ++t) {
-                dt += sle[t];
-                tdt += stle[t];
-                sx += scx[t];
-                sy += scy[t];
-                sz += scz[t];
-            }
-            dLe_total[2 * i + l] = dt;
-            TdLe_total[2 * i + l] = tdt;
-            cs_sum[6 * i + 3 * l] = sx;
-            cs_sum[6 * i + 3 * l + 1] = sy;
-            cs_sum[6 * i + 3 * l + 2] = sz;
-            stot[tid][l] = dt;
+    // five sums per particle and layer, a thread each, every one in bond order
+    for (int q = tid; q < 10 * np; q += 64) {
+        const int pl = q / 5, k = q - 5 * pl, p = pl >> 1, l = pl & 1;
+        const int64_t i = p0 + p;
+        const double *v = k == 0 ? sle : (k == 1 ? stle : (k == 2 ? scx : (k == 3 ? scy : scz)));
+        double x = 0;
+        for (int t = (l == 0 ? sbp[p] : ssp[p]) - B0; t < (l == 0 ? ssp[p] : sbp[p + 1]) - B0; ++t) x += v[t];
+        if (k == 0) {
+            dLe_total[2 * i + l] = x;
+            stot[p][l] = x;
+        } else if (k == 1) {
+            TdLe_total[2 * i + l] = x;
+        } else {
+            cs_sum[6 * i + 3 * l + k - 2] = x;
         }
     }
     __syncthreads();
@@ -122,22 +119,36 @@ __global__ __launch_bounds__(64) void k_geometry_force(
     }
 }
 
-// Bond forces only (geometry already current); used after a damage update.
-__global__ __launch_bounds__(256) void k_bond_force(int64_t n, int model, const int32_t *__restrict__ bptr,
-                                                     const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
-                                                     const double *__restrict__ Kn, const double *__restrict__ Tv,
-                                                     const double *__restrict__ dLe, const double *__restrict__ dLe_total,
-                                                     const double *__restrict__ damage, double *__restrict__ bforce,
-                                                     double *__restrict__ bdamage) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int b0 = bptr[i], bm = bsplit[i], b1 = bptr[i + 1];
-    const double Di = damage[i];
-    for (int b = b0; b < b1; ++b) {
-        double f = 2. * Kn[b] * dLe[b] + 2. * Tv[b] * dLe_total[2 * i + (b < bm ? 0 : 1)];
+// Bond forces only (geometry already current). Bound by memory: six per-bond arrays, read and written in
+// order by the same workgroups as k_geometry_force, a lane per bond. A thread per particle walking its own
+// bonds spread every load over 64 lines: this pass and k_particle_force together 439 -> 117 us at SC 64^3,
+// 39.8 -> 27.6 at FCC 20^3, 14.4 -> 10.3 at a hexagon plate of 1,007 particles.
+__global__ __launch_bounds__(64) void k_bond_force(int64_t n, int model, const int32_t *__restrict__ bptr,
+                                                    const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
+                                                    const double *__restrict__ Kn, const double *__restrict__ Tv,
+                                                    const double *__restrict__ dLe, const double *__restrict__ dLe_total,
+                                                    const double *__restrict__ damage, double *__restrict__ bforce,
+                                                    double *__restrict__ bdamage) {
+    __shared__ int sbp[GP + 1], ssp[GP];
+    __shared__ double stot[GP][2];
+    __shared__ uint8_t own[GP * LPM_MAXB];
+    const int tid = threadIdx.x;
+    const int64_t p0 = (int64_t)blockIdx.x * GP;
+    const int np = (int)((n - p0) < GP ? (n - p0) : GP);
+    if (tid <= np) sbp[tid] = bptr[p0 + tid];
+    if (tid < np) ssp[tid] = bsplit[p0 + tid];
+    if (tid < 2 * np) stot[tid >> 1][tid & 1] = dLe_total[2 * p0 + tid];
+    __syncthreads();
+    const int B0 = sbp[0], nbk = sbp[np] - B0, p = tid >> 3;
+    if (p < np)
+        for (int b = sbp[p] + (tid & 7); b < sbp[p + 1]; b += 8) own[b - B0] = (uint8_t)p;
+    __syncthreads();
+    for (int t = tid; t < nbk; t += 64) {
+        const int b = B0 + t, q = own[t];
+        double f = 2. * Kn[b] * dLe[b] + 2. * Tv[b] * stot[q][b < ssp[q] ? 0 : 1];
         double bd = bdamage[b];
         if (model != ELASTIC) {
-            bd = dmax(bd, dmax(Di, damage[p2[b]]));
+            bd = dmax(bd, dmax(damage[p0 + q], damage[p2[b]]));
             bdamage[b] = bd;
         }
         f *= (1.0 - bd);
@@ -147,8 +158,8 @@ __global__ __launch_bounds__(256) void k_bond_force(int64_t n, int model, const 
 
 // Particle::updateParticleForce / updateParticleStress / updateParticleDamageVisual
 // (particle.h:150-161, 197-240); the reverse bond comes from the precomputed opp[]. Same
-// workgroup layout as k_geometry_force: lane-per-bond loads into LDS, then per-particle sums in
-// bond order.
+// workgroup layout as k_geometry_force: lane-per-bond loads into LDS, then the ten sums of each
+// particle, a thread each, in bond order.
 __global__ __launch_bounds__(64) void k_particle_force(int64_t n, double volume, int nneighbors,
                                                         const int32_t *__restrict__ bptr, const int32_t *__restrict__ opp,
                                                         const double *__restrict__ cs, const double *__restrict__ dis,
@@ -174,38 +185,31 @@ __global__ __launch_bounds__(64) void k_particle_force(int64_t n, double volume,
         sbd[t] = bdamage[b];
     }
     __syncthreads();
-    if (tid >= np) return;
-    const int64_t i = p0 + tid;
-    const int lo = sbp[tid] - B0, hi = sbp[tid + 1] - B0;
-    const int nb = hi - lo;
-    const double V_m = volume * nb / nneighbors;
-    double P0 = 0., P1 = 0., P2 = 0.;
-    double s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0, dv = 0;
-    for (int t = lo; t < hi; ++t) {
-        const double ff = sff[t];
-        const double cx = scx[t], cy = scy[t], cz = scz[t];
-        P0 += cx * 0.5 * ff;
-        P1 += cy * 0.5 * ff;
-        P2 += cz * 0.5 * ff;
-        const double w = 0.5 / V_m * sdis[t] * 0.5 * ff;
-        s0 += w * cx * cx;
-        s1 += w * cy * cy;
-        s2 += w * cz * cz;
-        s3 += w * cy * cz;
-        s4 += w * cx * cz;
-        s5 += w * cx * cy;
-        dv += sbd[t];
+    // ten sums per particle, a thread each, every one in bond order
+    for (int q = tid; q < 10 * np; q += 64) {
+        const int p = q / 10, k = q - 10 * p;
+        const int64_t i = p0 + p;
+        const int lo = sbp[p] - B0, hi = sbp[p + 1] - B0, nb = hi - lo;
+        double x = 0.;
+        if (k < 3) {
+            const double *c = k == 0 ? scx : (k == 1 ? scy : scz);
+            for (int t = lo; t < hi; ++t) x += c[t] * 0.5 * sff[t];
+            Pin[3 * i + k] = x;
+        } else if (k < 9) {
+            // stress components xx yy zz yz xz xy
+            const double V_m = volume * nb / nneighbors;
+            const double *a = k == 3 || k == 7 || k == 8 ? scx : (k == 4 || k == 6 ? scy : scz);
+            const double *b = k == 3 ? scx : (k == 4 || k == 8 ? scy : scz);
+            for (int t = lo; t < hi; ++t) {
+                const double w = 0.5 / V_m * sdis[t] * 0.5 * sff[t];
+                x += w * a[t] * b[t];
+            }
+            stress[6 * i + k - 3] = x;
+        } else {
+            for (int t = lo; t < hi; ++t) x += sbd[t];
+            damage_visual[i] = x / (double)nb;
+        }
     }
-    Pin[3 * i] = P0;
-    Pin[3 * i + 1] = P1;
-    Pin[3 * i + 2] = P2;
-    stress[6 * i] = s0;
-    stress[6 * i + 1] = s1;
-    stress[6 * i + 2] = s2;
-    stress[6 * i + 3] = s3;
-    stress[6 * i + 4] = s4;
-    stress[6 * i + 5] = s5;
-    damage_visual[i] = dv / (double)nb;
 }
 
 // Solver::updateRR (solver.h:108-128) with the squared norms of residual and reaction.
@@ -1535,7 +1539,7 @@ int launch_geometry_force(lpm_ctx *c, bool force) {
 }
 
 int launch_bond_force(lpm_ctx *c) {
-    hipLaunchKernelGGL(k_bond_force, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->model, c->bptr, c->bsplit,
+    hipLaunchKernelGGL(k_bond_force, dim3(blocks_for(c->n, GP)), dim3(64), 0, c->stream, c->n, c->model, c->bptr, c->bsplit,
                        c->p2, c->Kn, c->Tv, c->dLe, c->dLe_total, c->damage, c->bforce, c->bdamage);
     return check_launch(c, "k_bond_force");
 }
