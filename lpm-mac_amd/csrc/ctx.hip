@@ -20,6 +20,16 @@ int lpm_fail(lpm_ctx *c, int code, const std::string &msg) {
     return code;
 }
 
+// the arrays of s in one allocation that the context keeps, zeroed on its stream
+int slab_alloc(lpm_ctx *c, Slab &s, bool zero) {
+    void *base = nullptr;
+    hipError_t e = s.alloc(&base);
+    if (e != hipSuccess) return lpm_fail(c, LPM_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    c->slabs.push_back(base);
+    if (zero) LPM_HIP(c, hipMemsetAsync(base, 0, s.bytes, c->stream));
+    return LPM_OK;
+}
+
 namespace {
 
 // ---------------------------------------------------------------- BC kernels
@@ -200,13 +210,14 @@ Field field(lpm_ctx *c, const std::string &w) {
     return {nullptr, 0, -1, false};
 }
 
-template <typename T>
-int dalloc(lpm_ctx *c, T **p, int64_t count) {
-    hipError_t e = hipMalloc((void **)p, sizeof(T) * (count > 0 ? count : 1));
-    if (e != hipSuccess) return lpm_fail(c, LPM_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-    e = hipMemsetAsync(*p, 0, sizeof(T) * (count > 0 ? count : 1), c->stream);
-    if (e != hipSuccess) return lpm_fail(c, LPM_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
-    return LPM_OK;
+// what FatigueHCF starts from (particle_fatigue_hcf.h:24-25, 229-236); all else starts at zero
+__global__ __launch_bounds__(256) void k_hcf_init(int64_t n, double *__restrict__ sv, double *__restrict__ sv_last,
+                                                  double *__restrict__ mat) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    sv[LPM_NSV * i + 1] = sv_last[LPM_NSV * i + 1] = (double)INT_MAX;
+    mat[LPM_NMAT * i + 5] = 1.0;
+    mat[LPM_NMAT * i + 6] = 1.108;
 }
 
 int copy_d2d(lpm_ctx *c, void *dst, const void *src, size_t bytes) {
@@ -825,7 +836,8 @@ static int create(const lpm_topology *t, const lpm_cut *cuts, int32_t ncut, lpm_
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream) == hipSuccess;
     };
     const double *x = t->xyz;
-#define AL(ptr, cnt) if ((rc = dalloc(c, &c->ptr, (cnt)))) return fail(rc)
+    Slab slab;
+#define AL(ptr, cnt) slab.add(&c->ptr, (cnt))
     // ---- per-particle arrays
     AL(xyz, 3 * n); AL(xyz0, 3 * n); AL(xyz_last, 3 * n); AL(Pin, 3 * n); AL(Pex, 3 * n); AL(stress, 6 * n);
     AL(damage, n); AL(damage_last, n); AL(damage_visual, n); AL(Ddot_local, n); AL(Ddot_nonlocal, n); AL(nonlocal_L, n);
@@ -833,11 +845,13 @@ static int create(const lpm_topology *t, const lpm_cut *cuts, int32_t ncut, lpm_
     AL(dLe_total, 2 * n); AL(TdLe_total, 2 * n); AL(cs_sum, 6 * n); AL(type, n); AL(cons, 3 * n);
     AL(residual, c->dim * n); AL(disp, c->dim * n); AL(diag64, c->dim * n);
     AL(scal, SC_COUNT); AL(counter, 8); AL(iflag, 8);
-    if (!(up(c->xyz, x, sizeof(double) * 3 * n) && up(c->xyz0, x, sizeof(double) * 3 * n) &&
-          up(c->xyz_last, x, sizeof(double) * 3 * n))) {
+    if ((rc = slab_alloc(c, slab, true))) return fail(rc);
+    if (!up(c->xyz, x, sizeof(double) * 3 * n)) {
         c->err = "position upload failed";
         return fail(LPM_E_HIP);
     }
+    if ((rc = copy_d2d(c, c->xyz0, c->xyz, sizeof(double) * 3 * n)) || (rc = copy_d2d(c, c->xyz_last, c->xyz, sizeof(double) * 3 * n)))
+        return fail(rc);
     // ---- bonds: Bond(p1, p2, layer, dis) (bond.h:61-73), reverse bonds, 2-hop bookkeeping
     if (search) {
         if ((rc = device_topology(c, x, cuts, ncut))) return fail(rc);
@@ -856,8 +870,10 @@ static int create(const lpm_topology *t, const lpm_cut *cuts, int32_t ncut, lpm_
             }
             c->asm_hops = std::max(c->asm_hops, hops);
         }
+        slab = Slab();
         AL(bptr, n + 1); AL(bsplit, n); AL(p2, nbond); AL(opp, nbond); AL(nbarr, n);
         AL(dis0, nbond); AL(dis, nbond); AL(dis_last, nbond); AL(cs, 3 * nbond);
+        if ((rc = slab_alloc(c, slab, false))) return fail(rc);
         std::vector<double> dis0(nbond), cs(3 * nbond);
         std::vector<int32_t> nb(n);
         for (int64_t i = 0; i < n; ++i) {
@@ -880,29 +896,24 @@ static int create(const lpm_topology *t, const lpm_cut *cuts, int32_t ncut, lpm_
         if (!ok) { c->err = "topology upload failed"; return fail(LPM_E_HIP); }
     }
     // ---- per-bond state
+    c->partial_cap = std::max({blocks_for(n * c->dim, 256), blocks_for(n, 4), blocks_for(n, 256), 1});
+    slab = Slab();
     AL(dLe, nbond); AL(dLp, nbond); AL(dLp_last, nbond);
     AL(bstrain, nbond); AL(Kn, nbond); AL(Tv, nbond); AL(bforce, nbond); AL(bforce_last, nbond);
     AL(bdamage, nbond); AL(bdamage_last, nbond);
-#undef AL
-    c->partial_cap = std::max({blocks_for(n * c->dim, 256), blocks_for(n, 4), blocks_for(n, 256), 1});
     // CG: (||r||^2, gamma) partials in two parity slots + the SpMV's delta partials
-    if ((rc = dalloc(c, &c->partial, 5 * (int64_t)c->partial_cap))) return fail(rc);
+    AL(partial, 5 * (int64_t)c->partial_cap);
+#undef AL
+    if ((rc = slab_alloc(c, slab, true))) return fail(rc);
     if (hipHostMalloc((void **)&c->h_scal, sizeof(double) * (SC_COUNT + 2)) != hipSuccess ||
         hipHostMalloc((void **)&c->h_iflag, sizeof(int32_t) * 8) != hipSuccess) {
         c->err = "hipHostMalloc failed";
         return fail(LPM_E_NOMEM);
     }
-    std::vector<double> sv(LPM_NSV * n, 0.0), mat(LPM_NMAT * n, 0.0);
-    if (c->model == LPM_FATIGUE_HCF)  // particle_fatigue_hcf.h:24-25, 229-236
-        for (int64_t i = 0; i < n; ++i) {
-            sv[LPM_NSV * i + 1] = (double)INT_MAX;
-            mat[LPM_NMAT * i + 5] = 1.0;
-            mat[LPM_NMAT * i + 6] = 1.108;
-        }
-    const bool ok = up(c->sv, sv.data(), sizeof(double) * LPM_NSV * n) &&
-                    up(c->sv_last, sv.data(), sizeof(double) * LPM_NSV * n) &&
-                    up(c->mat, mat.data(), sizeof(double) * LPM_NMAT * n);
-    if (!ok) { c->err = "state upload failed"; return fail(LPM_E_HIP); }
+    if (c->model == LPM_FATIGUE_HCF) {
+        hipLaunchKernelGGL(k_hcf_init, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, c->sv, c->sv_last, c->mat);
+        if (hipGetLastError() != hipSuccess) { c->err = "k_hcf_init"; return fail(LPM_E_HIP); }
+    }
     if ((rc = launch_pattern(c))) return fail(rc);
     if (hipStreamSynchronize(c->stream) != hipSuccess) { c->err = "sync failed"; return fail(LPM_E_HIP); }
     *out = c;
@@ -918,15 +929,10 @@ int lpm_create_cut(const lpm_topology *t, const lpm_cut *cuts, int32_t ncut, lpm
 int lpm_destroy(lpm_ctx *c) {
     if (!c) return LPM_OK;
     if (c->stream) hipStreamSynchronize(c->stream);
-    void *ptrs[] = {c->bptr, c->bsplit, c->p2, c->opp, c->nbarr, c->cptr, c->cidx, c->tslot, c->nlptr, c->nlidx, c->xyz,
-                    c->xyz0, c->xyz_last, c->Pin, c->Pex, c->stress, c->damage, c->damage_last, c->damage_visual,
-                    c->Ddot_local, c->Ddot_nonlocal, c->nonlocal_L, c->sv, c->sv_last, c->mat, c->dLe_total, c->TdLe_total,
-                    c->cs_sum, c->type, c->cons, c->dis0, c->dis, c->dis_last, c->dLe, c->dLp, c->dLp_last, c->bstrain, c->Kn,
-                    c->Tv, c->cs, c->bforce, c->bforce_last, c->bdamage, c->bdamage_last, c->residual, c->disp, c->diag64,
-                    c->aval, c->invdiag, c->v_x, c->v_r, c->v_u, c->v_p, c->v_s, c->v_w, c->scal, c->partial, c->counter, c->iflag, c->sp, c->scol,
-                    c->scol16, c->pl_row, c->pl_slot, c->pl_rng, c->pl_b3, c->pl_own,
-                    c->spec_of, c->spec_w, c->spec_blk, c->spec_first_d, c->spec_part, c->xyz_prev, c->xyz_prev2,
-                    c->elim};
+    void *ptrs[] = {c->tslot, c->nlptr, c->nlidx, c->aval, c->invdiag, c->v_x, c->v_r, c->v_u, c->v_p, c->v_s, c->v_w,
+                    c->scol16, c->pl_row, c->pl_slot, c->pl_rng, c->pl_b3, c->pl_own, c->spec_of, c->spec_w, c->spec_blk,
+                    c->spec_first_d, c->spec_part, c->xyz_prev, c->xyz_prev2, c->elim};
+    for (void *p : c->slabs) hipFree(p);
     for (void *p : ptrs)
         if (p) hipFree(p);
     dump_free(c);

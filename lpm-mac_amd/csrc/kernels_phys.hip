@@ -2074,24 +2074,24 @@ int device_topology(lpm_ctx *c, const double *xyz_host, const lpm_cut *cuts_host
     for (int k = 0; k < 3; ++k) nc[k] = std::max<int64_t>(1, (int64_t)std::floor((hi[k] - lo[k]) / h) + 1);
     const int64_t ncell = nc[0] * nc[1] * nc[2];
     if (ncell >= 0x7fffffffLL) return lpm_fail(c, LPM_E_LIMIT, "bond search grid too large");
-    int32_t *pcell = nullptr, *count = nullptr, *head = nullptr, *items = nullptr, *tmp0 = nullptr, *tmp1 = nullptr,
-            *cnt = nullptr, *flag = nullptr;
+    int32_t *pcell, *count, *head, *items, *tmp0, *tmp1, *cnt, *flag;
     lpm_cut *dcuts = nullptr;
+    void *scratch_base = nullptr;
     auto cleanup = [&]() {
-        void *ps[] = {pcell, count, head, items, tmp0, tmp1, cnt, flag, dcuts};
-        for (void *q : ps)
-            if (q) hipFree(q);
+        if (scratch_base) hipFree(scratch_base);
     };
-    auto al = [&](int32_t **p, int64_t cntv) { return hipMalloc(p, sizeof(int32_t) * std::max<int64_t>(cntv, 1)) == hipSuccess; };
-    if (!al(&pcell, n) || !al(&count, ncell) || !al(&head, ncell + 1) || !al(&items, n) || !al(&tmp0, n * LPM_MAXB) ||
-        !al(&tmp1, n * LPM_MAXB) || !al(&cnt, 2 * n) || !al(&flag, 4)) {
-        cleanup();
-        return lpm_fail(c, LPM_E_NOMEM, "bond search scratch");
-    }
-    if (ncut > 0) {
-        if (hipMalloc(&dcuts, sizeof(lpm_cut) * ncut) != hipSuccess) { cleanup(); return lpm_fail(c, LPM_E_NOMEM, "cuts"); }
-        hipMemcpyAsync(dcuts, cuts_host, sizeof(lpm_cut) * ncut, hipMemcpyHostToDevice, c->stream);
-    }
+    Slab tmp;
+    tmp.add(&pcell, n);
+    tmp.add(&count, ncell);
+    tmp.add(&head, ncell + 1);
+    tmp.add(&items, n);
+    tmp.add(&tmp0, n * LPM_MAXB);
+    tmp.add(&tmp1, n * LPM_MAXB);
+    tmp.add(&cnt, 2 * n);
+    tmp.add(&flag, 4);
+    if (ncut > 0) tmp.add(&dcuts, ncut);
+    if (tmp.alloc(&scratch_base) != hipSuccess) return lpm_fail(c, LPM_E_NOMEM, "bond search scratch");
+    if (ncut > 0) hipMemcpyAsync(dcuts, cuts_host, sizeof(lpm_cut) * ncut, hipMemcpyHostToDevice, c->stream);
     int rc = LPM_OK;
     std::vector<int32_t> h_count(ncell), h_head(ncell + 1, 0), h_cnt(2 * n);
     hipMemsetAsync(count, 0, sizeof(int32_t) * ncell, c->stream);
@@ -2132,14 +2132,17 @@ int device_topology(lpm_ctx *c, const double *xyz_host, const lpm_cut *cuts_host
     c->gp_bonds = 0;
     for (int64_t p0 = 0; p0 < n; p0 += LPM_BOND_GP)
         c->gp_bonds = std::max<int>(c->gp_bonds, bp[std::min<int64_t>(n, p0 + LPM_BOND_GP)] - bp[p0]);
-#define ALT(ptr, cntv)                                                                                          \
-    if (hipMalloc(&c->ptr, sizeof(*c->ptr) * std::max<int64_t>((cntv), 1)) != hipSuccess) {                     \
-        cleanup();                                                                                               \
-        return lpm_fail(c, LPM_E_NOMEM, "topology arrays");                                                      \
-    }
-    ALT(bptr, n + 1); ALT(bsplit, n); ALT(p2, tot); ALT(opp, tot); ALT(nbarr, n);
-    ALT(dis0, tot); ALT(dis, tot); ALT(dis_last, tot); ALT(cs, 3 * tot);
-#undef ALT
+    Slab slab;
+    slab.add(&c->bptr, n + 1);
+    slab.add(&c->bsplit, n);
+    slab.add(&c->p2, tot);
+    slab.add(&c->opp, tot);
+    slab.add(&c->nbarr, n);
+    slab.add(&c->dis0, tot);
+    slab.add(&c->dis, tot);
+    slab.add(&c->dis_last, tot);
+    slab.add(&c->cs, 3 * tot);
+    if ((rc = slab_alloc(c, slab, false))) { cleanup(); return rc; }
     hipMemcpyAsync(c->bptr, bp.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice, c->stream);
     hipMemcpyAsync(c->bsplit, bs.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, c->stream);
     hipLaunchKernelGGL(k_bond_compact, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, (const int32_t *)c->bptr,
@@ -2181,15 +2184,6 @@ int launch_pattern(lpm_ctx *c) {
     }
     c->nconn = cp[c->n];
     c->maxconn = maxc;
-    LPM_HIP(c, hipMalloc(&c->cptr, sizeof(int32_t) * (c->n + 1)));
-    LPM_HIP(c, hipMalloc(&c->cidx, sizeof(int32_t) * (c->nconn > 0 ? c->nconn : 1)));
-    LPM_HIP(c, hipMemcpyAsync(c->cptr, cp.data(), sizeof(int32_t) * (c->n + 1), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_pattern, dim3((unsigned)c->n), dim3(256), 0, c->stream, c->n, c->bptr, c->bsplit, c->p2, counts,
-                       (const int32_t *)c->cptr, c->cidx, c->iflag);
-    rc = check_launch(c, "k_pattern(fill)");
-    LPM_HIP(c, hipStreamSynchronize(c->stream));
-    hipFree(counts);
-    if (rc) return rc;
     // SELL-64 slice offsets: slice k covers rows 64k..64k+63 and is as wide as its longest row
     c->nslice = (c->n + 63) / 64;
     std::vector<int64_t> sp(c->nslice + 1, 0);
@@ -2199,8 +2193,19 @@ int launch_pattern(lpm_ctx *c) {
         sp[k + 1] = sp[k] + 64LL * W;
     }
     c->nslots = sp[c->nslice];
-    LPM_HIP(c, hipMalloc(&c->sp, sizeof(int64_t) * (c->nslice + 1)));
-    LPM_HIP(c, hipMalloc(&c->scol, sizeof(int32_t) * (c->nslots > 0 ? c->nslots : 1)));
+    Slab slab;
+    slab.add(&c->cptr, c->n + 1);
+    slab.add(&c->cidx, c->nconn);
+    slab.add(&c->sp, c->nslice + 1);
+    slab.add(&c->scol, c->nslots);
+    if ((rc = slab_alloc(c, slab, false))) { hipFree(counts); return rc; }
+    LPM_HIP(c, hipMemcpyAsync(c->cptr, cp.data(), sizeof(int32_t) * (c->n + 1), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_pattern, dim3((unsigned)c->n), dim3(256), 0, c->stream, c->n, c->bptr, c->bsplit, c->p2, counts,
+                       (const int32_t *)c->cptr, c->cidx, c->iflag);
+    rc = check_launch(c, "k_pattern(fill)");
+    LPM_HIP(c, hipStreamSynchronize(c->stream));
+    hipFree(counts);
+    if (rc) return rc;
     LPM_HIP(c, hipMemcpyAsync(c->sp, sp.data(), sizeof(int64_t) * (c->nslice + 1), hipMemcpyHostToDevice, c->stream));
     hipLaunchKernelGGL(k_sell_cols, dim3(blocks_for(c->n, 256)), dim3(256), 0, c->stream, c->n, c->cptr, c->cidx, c->sp, c->scol);
     rc = check_launch(c, "k_sell_cols");
@@ -2282,17 +2287,16 @@ static int nonlocal_search_cells(lpm_ctx *c, double ratio, bool *done) {
         h *= 1.5;
     }
     if (ncell >= 0x7fffffffLL) return LPM_OK;
-    int32_t *pcell = nullptr, *count = nullptr, *head = nullptr, *items = nullptr, *counts = nullptr;
-    auto cleanup = [&]() {
-        void *ps[] = {pcell, count, head, items, counts};
-        for (void *q : ps)
-            if (q) hipFree(q);
-    };
-    auto al = [&](int32_t **q, int64_t m) { return hipMalloc(q, sizeof(int32_t) * std::max<int64_t>(m, 1)) == hipSuccess; };
-    if (!al(&pcell, n) || !al(&count, ncell) || !al(&head, ncell + 1) || !al(&items, n) || !al(&counts, n)) {
-        cleanup();
-        return lpm_fail(c, LPM_E_NOMEM, "nonlocal search scratch");
-    }
+    int32_t *pcell, *count, *head, *items, *counts;
+    void *scratch_base = nullptr;
+    auto cleanup = [&]() { hipFree(scratch_base); };
+    Slab tmp;
+    tmp.add(&pcell, n);
+    tmp.add(&count, ncell);
+    tmp.add(&head, ncell + 1);
+    tmp.add(&items, n);
+    tmp.add(&counts, n);
+    if (tmp.alloc(&scratch_base) != hipSuccess) return lpm_fail(c, LPM_E_NOMEM, "nonlocal search scratch");
     int rc = LPM_OK;
     auto hip_ok = [&](hipError_t e, const char *what) {
         if (e == hipSuccess) return true;
