@@ -121,8 +121,8 @@ __global__ __launch_bounds__(64) void k_geometry_force(
 
 // Bond forces only (geometry already current). Bound by memory: six per-bond arrays, read and written in
 // order by the same workgroups as k_geometry_force, a lane per bond. A thread per particle walking its own
-// bonds spread every load over 64 lines: this pass and k_particle_force together 439 -> 117 us at SC 64^3,
-// 39.8 -> 27.6 at FCC 20^3, 14.4 -> 10.3 at a hexagon plate of 1,007 particles.
+// bonds spread every load over 64 lines: this pass and k_particle_force together 439 -> 101 us at SC 64^3,
+// 39.8 -> 25.3 at FCC 20^3, 14.4 -> 8.4 at a hexagon plate of 1,007 particles.
 __global__ __launch_bounds__(64) void k_bond_force(int64_t n, int model, const int32_t *__restrict__ bptr,
                                                     const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
                                                     const double *__restrict__ Kn, const double *__restrict__ Tv,
@@ -158,8 +158,9 @@ __global__ __launch_bounds__(64) void k_bond_force(int64_t n, int model, const i
 
 // Particle::updateParticleForce / updateParticleStress / updateParticleDamageVisual
 // (particle.h:150-161, 197-240); the reverse bond comes from the precomputed opp[]. Same
-// workgroup layout as k_geometry_force: lane-per-bond loads into LDS, then the ten sums of each
-// particle, a thread each, in bond order.
+// workgroup layout as k_geometry_force: lane-per-bond loads into LDS, then per-particle sums in
+// bond order, here a thread per particle: a thread per sum read the staged bonds ten times and made a load path
+// at SC 64^3 0.4% slower.
 __global__ __launch_bounds__(64) void k_particle_force(int64_t n, double volume, int nneighbors,
                                                         const int32_t *__restrict__ bptr, const int32_t *__restrict__ opp,
                                                         const double *__restrict__ cs, const double *__restrict__ dis,
@@ -185,31 +186,38 @@ __global__ __launch_bounds__(64) void k_particle_force(int64_t n, double volume,
         sbd[t] = bdamage[b];
     }
     __syncthreads();
-    // ten sums per particle, a thread each, every one in bond order
-    for (int q = tid; q < 10 * np; q += 64) {
-        const int p = q / 10, k = q - 10 * p;
-        const int64_t i = p0 + p;
-        const int lo = sbp[p] - B0, hi = sbp[p + 1] - B0, nb = hi - lo;
-        double x = 0.;
-        if (k < 3) {
-            const double *c = k == 0 ? scx : (k == 1 ? scy : scz);
-            for (int t = lo; t < hi; ++t) x += c[t] * 0.5 * sff[t];
-            Pin[3 * i + k] = x;
-        } else if (k < 9) {
-            // stress components xx yy zz yz xz xy
-            const double V_m = volume * nb / nneighbors;
-            const double *a = k == 3 || k == 7 || k == 8 ? scx : (k == 4 || k == 6 ? scy : scz);
-            const double *b = k == 3 ? scx : (k == 4 || k == 8 ? scy : scz);
-            for (int t = lo; t < hi; ++t) {
-                const double w = 0.5 / V_m * sdis[t] * 0.5 * sff[t];
-                x += w * a[t] * b[t];
-            }
-            stress[6 * i + k - 3] = x;
-        } else {
-            for (int t = lo; t < hi; ++t) x += sbd[t];
-            damage_visual[i] = x / (double)nb;
-        }
+    if (tid >= np) return;
+    const int64_t i = p0 + tid;
+    const int lo = sbp[tid] - B0, hi = sbp[tid + 1] - B0;
+    const int nb = hi - lo;
+    const double V_m = volume * nb / nneighbors;
+    double P0 = 0., P1 = 0., P2 = 0.;
+    double s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0, dv = 0;
+    for (int t = lo; t < hi; ++t) {
+        const double ff = sff[t];
+        const double cx = scx[t], cy = scy[t], cz = scz[t];
+        P0 += cx * 0.5 * ff;
+        P1 += cy * 0.5 * ff;
+        P2 += cz * 0.5 * ff;
+        const double w = 0.5 / V_m * sdis[t] * 0.5 * ff;
+        s0 += w * cx * cx;
+        s1 += w * cy * cy;
+        s2 += w * cz * cz;
+        s3 += w * cy * cz;
+        s4 += w * cx * cz;
+        s5 += w * cx * cy;
+        dv += sbd[t];
     }
+    Pin[3 * i] = P0;
+    Pin[3 * i + 1] = P1;
+    Pin[3 * i + 2] = P2;
+    stress[6 * i] = s0;
+    stress[6 * i + 1] = s1;
+    stress[6 * i + 2] = s2;
+    stress[6 * i + 3] = s3;
+    stress[6 * i + 4] = s4;
+    stress[6 * i + 5] = s5;
+    damage_visual[i] = dv / (double)nb;
 }
 
 // Solver::updateRR (solver.h:108-128) with the squared norms of residual and reaction.
