@@ -4,7 +4,7 @@
 //
 // What bounds a solve of a small or middle-sized system is not the matrix but the chain of dependent
 // steps: five kernels of 3-10 us per iteration whose work is a microsecond or two each, and every
-// launch starts with cold caches. Here a workgroup of 16 wavefronts owns the same 64-row slices for
+// launch starts with cold caches. Here a workgroup of eight wavefronts owns the same 64-row slices for
 // the whole solve. Its threads hold their rows' x, r, p, s and diagonal in registers, its part of the
 // matrix stays in the XCD's L2, and only these travel between workgroups, once per iteration
 // each: the aggregates' shares of P^T r and the coarse correction, the preconditioned residual u (read by the neighbours' SpMV)
