@@ -694,6 +694,7 @@ static int coarse_setup(lpm_ctx *c) {
 
 template <typename T, int D>
 static int coarse_rows_t(lpm_ctx *c) {
+    if (c->nra == 0) return LPM_OK;  // no bond, no column
     hipLaunchKernelGGL((k_coarse_rows<T, D>), dim3(blocks_for(c->nra, 64)), dim3(64), 0, c->stream, c->nra, c->cptr,
                        c->scol, c->sp, (const T *)c->aval, c->agg_of, c->agg_d, c->dofmask, c->ra_row, c->ra_id, c->cvbuf);
     return ck(c, "k_coarse_rows");
