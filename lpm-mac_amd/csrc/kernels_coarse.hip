@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void k_coarse_blocks(int64_t ncq, const int32_
 }
 
 // Blocked Gauss-Jordan inversion of the symmetrised Ac (SPD, so no pivoting), NB pivots per
-// block step, one launch per step (reading A_in, writing A_out, so no element is read after
+// block step, one or three launches per step (reading A_in, writing A_out, so no element is read after
 // another thread wrote it). A coarse DoF whose row is zero (an aggregate whose DoFs are all
 // eliminated) is set to the identity before and to zero after, so it receives no correction.
 // A coarse DoF whose pivot (its Schur complement against the pivots before it) falls to
@@ -178,11 +178,49 @@ __global__ __launch_bounds__(256) void k_coarse_dead(int ncoarse, int M, const i
     }
 }
 
-// Dinv = A[K,K]^-1 of the nb x nb pivot block in D by Gauss-Jordan with the pivot drop described
-// above, by one wavefront: lane (h, i) holds columns 16h .. 16h+15 of row i in registers, and each pivot's row
-// and column pass through LDS without a barrier. 32 pivots take 5 us; a workgroup of one
-// thread per element with two barriers per pivot took 16 us. Dinv is NB x NB, zero outside nb x nb and in the rows and
-// columns of dropped pivots.
+// Dinv = A[K,K]^-1 of every group (one workgroup each) by Gauss-Jordan in LDS, with the pivot drop
+// described above: the first of the three kernels of a step, and the start of the fused steps. Dinv is
+// stored NB x NB (row stride NB), zero outside nb x nb and in the rows and columns of dropped pivots.
+__global__ __launch_bounds__(1024) void k_gj_diag(int kb, const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
+                                                   const double *__restrict__ Ain, const double *__restrict__ odiag_all,
+                                                   uint8_t *__restrict__ dead_all, double *__restrict__ Dinv_all) {
+    __shared__ double D[GJ_NB][GJ_NB + 1];
+    __shared__ uint8_t skip[GJ_NB];
+    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
+    if (kb >= nc) return;  // this group's inversion has finished
+    const double *A = Ain + off[b];
+    const int nb = min(GJ_NB, nc - kb);
+    const int tid = threadIdx.x, i = tid / GJ_NB, j = tid % GJ_NB;  // blockDim = NB * NB
+    const bool in = i < nb && j < nb;
+    D[i][j] = in ? A[(int64_t)(kb + i) * nc + kb + j] : 0.0;
+    if (tid < GJ_NB) skip[tid] = 0;
+    __syncthreads();
+    for (int k = 0; k < nb; ++k) {
+        // every thread reads the same pivot, so the skip branch is uniform across the workgroup
+        const double pk = D[k][k];
+        if (!(pk > GJ_DROP * odiag_all[base + kb + k])) {
+            if (tid == 0) {
+                skip[k] = 1;
+                dead_all[base + kb + k] = 1;
+            }
+            continue;
+        }
+        const double rk = (j == k) ? 1.0 : D[k][j], ck = D[i][k];
+        __syncthreads();
+        if (in) {
+            const double p = 1.0 / pk;
+            if (i == k) D[i][j] = rk * p;
+            else D[i][j] = ((j == k) ? 0.0 : D[i][j]) - ck * rk * p;
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    Dinv_all[(int64_t)b * GJ_NB * GJ_NB + tid] = (in && !skip[i] && !skip[j]) ? D[i][j] : 0.0;
+}
+
+// The same inverse of the nb x nb pivot block in D by one wavefront, inside a fused step: lane (h, i) holds
+// columns 16h .. 16h+15 of row i in registers, and each pivot's row and column pass through LDS without a
+// barrier. It is the longest chain of a fused step: 16 of its 29 us with one block of 768 DoFs.
 __device__ __forceinline__ void gj_invert(const double (&D)[GJ_NB][GJ_NB + 1], double (*rc)[GJ_NB], int nb, const double *odiag,
                                           uint8_t *dead, double *Dinv) {
     const int lane = threadIdx.x & 63, h = lane >> 5, i = lane & 31;
@@ -226,24 +264,7 @@ __device__ __forceinline__ void gj_invert(const double (&D)[GJ_NB][GJ_NB + 1], d
     }
 }
 
-// The first pivot block of every group
-__global__ __launch_bounds__(64) void k_gj_diag(const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
-                                                const double *__restrict__ Ain, const double *__restrict__ odiag_all,
-                                                uint8_t *__restrict__ dead_all, double *__restrict__ Dinv_all) {
-    __shared__ double D[GJ_NB][GJ_NB + 1], rc[2][GJ_NB];
-    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
-    if (nc <= 0) return;
-    const double *A = Ain + off[b];
-    const int nb = min(GJ_NB, nc);
-    for (int e = threadIdx.x; e < GJ_NB * GJ_NB; e += 64) {
-        const int i = e / GJ_NB, j = e % GJ_NB;
-        D[i][j] = i < nb && j < nb ? A[(int64_t)i * nc + j] : 0.0;
-    }
-    __syncthreads();
-    gj_invert(D, rc, nb, odiag_all + base, dead_all + base, Dinv_all + (int64_t)b * GJ_NB * GJ_NB);
-}
-
-// Block step kb: the rank-NB update of the group's block, one 32 x 32 tile per workgroup (tiles are
+// A fused step kb: the rank-NB update of the group's block, one 32 x 32 tile per workgroup (tiles are
 // aligned with the pivot blocks, so a tile lies wholly inside or outside K in each direction). With
 // R = Dinv A[K, :]:
 //   tile in K x K:      Dinv
@@ -251,8 +272,17 @@ __global__ __launch_bounds__(64) void k_gj_diag(const int32_t *__restrict__ cb, 
 //   column tile in K:   -A[:,K] Dinv
 //   else:               A - A[:,K] R
 // Each workgroup forms its own 32 columns of R, and the one whose tile is the next pivot block inverts it
-// for the next step (into the other Dinv), so a step is one launch instead of three (inversion
-// 15.6, panel 7.0, update 12.8 us). A group whose inversion has finished is copied, so that every block ends in the same buffer.
+// for the next step (into the other Dinv). A group whose inversion has finished is copied, so that every
+// block ends in the same buffer.
+//
+// Forming R in every tile doubles the products of a step, so this pays only while a step is bound by its
+// launches and by the chain of 32 pivots, and not by the tiles. us per step with the first inverse, three kernels
+// and fused, blocks x DoFs (tiles): 1 x 432 (196) 31.0 and 26.4; 8 x 192 (288) 33.3 and 29.2; 1 x 768 (576) 35.2 and
+// 29.6; 24 x 147 (600) 35.5 and 30.5; 16 x 243 (1024) 38.7 and 38.9; 2 x 768 (1152) 39.6 and 35.8; 64 x 147 (1600) 43.0
+// and 43.1; 4 x 768 (2304) 49.7 and 49.5; 16 x 432 (3136) 54.2 and 55.7; 8 x 768 (4608) 66.1 and 75.0; 64 x 768
+// (36,864) 325 and 429. The line is drawn at eight tiles per CU.
+constexpr int64_t GJ_FUSED_TILES = 2048;
+
 __global__ __launch_bounds__(256) void k_gj_step(int kb, int T, const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
                                                   const double *__restrict__ Ain_all, double *__restrict__ Aout_all,
                                                   const double *__restrict__ Dinv_all, double *__restrict__ Dnext_all,
@@ -313,6 +343,90 @@ __global__ __launch_bounds__(256) void k_gj_step(int kb, int T, const int32_t *_
         if (threadIdx.x < 64)
             gj_invert(L, rc, min(GJ_NB, nc - i0), odiag_all + base + i0, dead_all + base + i0,
                       Dnext_all + (int64_t)b * GJ_NB * GJ_NB);
+    }
+}
+
+// Three kernels per step, part 2: the row panel Rt[j][k] = sum_m Dinv[k][m] A[kb+m][j] for j outside K
+// (zero for j in K), row stride NB; four threads per column j, eight k each, Dinv staged in LDS.
+__global__ __launch_bounds__(256) void k_gj_panel(int kb, const int32_t *__restrict__ cb, const int64_t *__restrict__ off,
+                                                   const double *__restrict__ Ain, const double *__restrict__ Dinv_all,
+                                                   double *__restrict__ Rt_all) {
+    __shared__ double Ds[GJ_NB][GJ_NB + 1];
+    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
+    if (kb >= nc || (int)(blockIdx.x * (blockDim.x >> 2)) >= nc) return;  // uniform over the workgroup
+    const double *Dinv = Dinv_all + (int64_t)b * GJ_NB * GJ_NB;
+    for (int e = threadIdx.x; e < GJ_NB * GJ_NB; e += blockDim.x) Ds[e / GJ_NB][e % GJ_NB] = Dinv[e];
+    __syncthreads();
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, j = t >> 2, k0 = (t & 3) * 8;
+    if (j >= nc) return;
+    const double *A = Ain + off[b];
+    const int nb = min(GJ_NB, nc - kb);
+    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (j < kb || j >= kb + nb)
+        for (int m = 0; m < nb; ++m) {
+            const double a = A[(int64_t)(kb + m) * nc + j];
+            for (int q = 0; q < 8; ++q) acc[q] += Ds[k0 + q][m] * a;
+        }
+    double *Rt = Rt_all + (int64_t)(base + j) * GJ_NB + k0;
+    for (int q = 0; q < 8; ++q) Rt[q] = acc[q];
+}
+
+// Three kernels per step, part 3: the rank-NB update of the group's block, one 32 x 32 tile per
+// workgroup (tiles are aligned with the pivot blocks, so a tile lies wholly inside or outside K
+// in each direction):
+//   tile in K x K:      Dinv
+//   row tile in K:      Rt^T
+//   column tile in K:   -A[:,K] Dinv
+//   else:               A - A[:,K] Rt^T
+// A group whose inversion has finished is copied, so that every block ends in the same buffer.
+__global__ __launch_bounds__(256) void k_gj_update(int kb, int T, const int32_t *__restrict__ cb,
+                                                    const int64_t *__restrict__ off, const double *__restrict__ Ain_all,
+                                                    double *__restrict__ Aout_all, const double *__restrict__ Dinv_all,
+                                                    const double *__restrict__ Rt_all) {
+    static_assert(GJ_NB == 32, "tiles are 32 x 32 pivot blocks");
+    __shared__ double L[32][33], R[32][33];
+    const int b = blockIdx.y, base = cb[b], nc = cb[b + 1] - base;
+    const int i0 = (blockIdx.x / T) * 32, j0 = (blockIdx.x % T) * 32;
+    if (i0 >= nc || j0 >= nc) return;  // uniform over the workgroup
+    const double *Ain = Ain_all + off[b];
+    double *Aout = Aout_all + off[b];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    if (kb >= nc) {
+        for (int q = 0; q < 4; ++q) {
+            const int i = i0 + ty + 8 * q, j = j0 + tx;
+            if (i < nc && j < nc) Aout[(int64_t)i * nc + j] = Ain[(int64_t)i * nc + j];
+        }
+        return;
+    }
+    const double *Dinv = Dinv_all + (int64_t)b * GJ_NB * GJ_NB, *Rt = Rt_all + (int64_t)base * GJ_NB;
+    const int nb = min(GJ_NB, nc - kb);
+    const bool ik = i0 == kb, jk = j0 == kb;
+    if (ik && jk) {
+        for (int q = 0; q < 4; ++q) {
+            const int ii = ty + 8 * q, i = i0 + ii, j = j0 + tx;
+            if (i < nc && j < nc) Aout[(int64_t)i * nc + j] = Dinv[ii * GJ_NB + tx];
+        }
+        return;
+    }
+    for (int e = threadIdx.x; e < 32 * 32; e += blockDim.x) {
+        const int r = e >> 5, m = e & 31;
+        // R[jj][m]: Rt rows j0.. (row tile in K and general case) or Dinv^T (column tile in K)
+        R[r][m] = jk ? Dinv[m * GJ_NB + r] : ((j0 + r < nc) ? Rt[(int64_t)(j0 + r) * GJ_NB + m] : 0.0);
+        L[r][m] = (!ik && i0 + r < nc && m < nb) ? Ain[(int64_t)(i0 + r) * nc + kb + m] : 0.0;
+    }
+    __syncthreads();
+    for (int q = 0; q < 4; ++q) {
+        const int ii = ty + 8 * q, i = i0 + ii, j = j0 + tx;
+        if (i >= nc || j >= nc) continue;
+        double v;
+        if (ik) {
+            v = R[tx][ii];
+        } else {
+            double s = 0.0;
+            for (int m = 0; m < 32; ++m) s += L[ii][m] * R[tx][m];
+            v = jk ? -s : Ain[(int64_t)i * nc + j] - s;
+        }
+        Aout[(int64_t)i * nc + j] = v;
     }
 }
 
@@ -655,12 +769,19 @@ static int coarse_setup(lpm_ctx *c) {
     LPM_HIP(c, hipMalloc(&c->ra_row, sizeof(int32_t) * std::max<size_t>(rid.size(), 1)));
     LPM_HIP(c, hipMalloc(&c->ra_id, sizeof(int32_t) * std::max<size_t>(rid.size(), 1)));
     LPM_HIP(c, hipMalloc(&c->cvbuf, sizeof(double) * M * M * std::max<size_t>(rid.size(), 1)));
-    // two ping-pong buffers of the packed blocks, two sets of the groups' NB x NB block inverses, the
-    // original diagonal and the dead-row flags
+    // two ping-pong buffers of the packed blocks, the groups' NB x NB block inverses (two sets for the fused
+    // steps, else one and the row panels), the original diagonal and the dead-row flags
+    int64_t tiles = 0;
+    for (int64_t s = 0; s < nsp; ++s) {
+        const int64_t t = (cb[s + 1] - cb[s] + GJ_NB - 1) / GJ_NB;
+        tiles += t * t;
+    }
+    c->gj_fused = tiles <= GJ_FUSED_TILES;
+    const size_t step_elems = (c->gj_fused ? 2 : 1) * (size_t)nsp * GJ_NB * GJ_NB + (c->gj_fused ? 0 : (size_t)nc * GJ_NB);
     c->ncgrp = (int)nsp;
     c->cgrp_nbmax = nbmax;
     c->ac_elems = off[nsp];
-    LPM_HIP(c, hipMalloc(&c->Ac, sizeof(double) * (2 * (size_t)c->ac_elems + 2 * (size_t)nsp * GJ_NB * GJ_NB + nc) + nc));
+    LPM_HIP(c, hipMalloc(&c->Ac, sizeof(double) * (2 * (size_t)c->ac_elems + step_elems + nc) + nc));
     LPM_HIP(c, hipMalloc(&c->cgrp_cb, sizeof(int32_t) * (nsp + 1)));
     LPM_HIP(c, hipMalloc(&c->cgrp_off, sizeof(int64_t) * (nsp + 1)));
     LPM_HIP(c, hipMalloc(&c->agg_grp, sizeof(int32_t) * std::max(nagg, 1)));
@@ -760,8 +881,9 @@ int coarse_prepare(lpm_ctx *c) {
         if ((rc = ck(c, "k_coarse_blocks"))) return rc;
     }
     const int64_t nd = (int64_t)G * GJ_NB * GJ_NB;
-    double *A0 = c->Ac, *A1 = c->Ac + ne, *Dinv = c->Ac + 2 * ne;  // two sets of block inverses
-    double *odiag = Dinv + 2 * nd;
+    double *A0 = c->Ac, *A1 = c->Ac + ne, *Dinv = c->Ac + 2 * ne;
+    double *Rt = Dinv + nd;  // the row panels, or the second set of block inverses
+    double *odiag = Rt + (c->gj_fused ? nd : (int64_t)nc * GJ_NB);
     uint8_t *dead = (uint8_t *)(odiag + nc);
     const int nsteps = (nbmax + GJ_NB - 1) / GJ_NB, T = nsteps;  // T x T tiles of 32 cover the largest block
     // every group's block in the same launches (grid y = group, x over the largest block)
@@ -772,14 +894,25 @@ int coarse_prepare(lpm_ctx *c) {
         hipLaunchKernelGGL(k_coarse_dead, dim3(blocks_for(nc, 4)), dim3(256), 0, c->stream, nc, M,
                            (const int32_t *)c->agg_grp, (const int32_t *)c->cgrp_cb, (const int64_t *)c->cgrp_off, A0, odiag,
                            dead);
-        hipLaunchKernelGGL(k_gj_diag, dim3(1, G), dim3(64), 0, c->stream, (const int32_t *)c->cgrp_cb,
-                           (const int64_t *)c->cgrp_off, (const double *)A0, (const double *)odiag, dead, Dinv);
+        auto diag = [&](int st, const double *A) {
+            hipLaunchKernelGGL(k_gj_diag, dim3(1, G), dim3(GJ_NB * GJ_NB), 0, c->stream, st * GJ_NB, (const int32_t *)c->cgrp_cb,
+                               (const int64_t *)c->cgrp_off, A, (const double *)odiag, dead, Dinv);
+        };
+        if (c->gj_fused) diag(0, A0);
         for (int st = 0; st < nsteps; ++st) {
             const double *Ain = (st & 1) ? A1 : A0;
             double *Aout = (st & 1) ? A0 : A1;
-            hipLaunchKernelGGL(k_gj_step, dim3(T * T, G), dim3(256), 0, c->stream, st * GJ_NB, T, (const int32_t *)c->cgrp_cb,
-                               (const int64_t *)c->cgrp_off, Ain, Aout, (const double *)(Dinv + (st & 1) * nd),
-                               Dinv + ((st + 1) & 1) * nd, (const double *)odiag, dead);
+            if (c->gj_fused) {
+                hipLaunchKernelGGL(k_gj_step, dim3(T * T, G), dim3(256), 0, c->stream, st * GJ_NB, T, (const int32_t *)c->cgrp_cb,
+                                   (const int64_t *)c->cgrp_off, Ain, Aout, (const double *)(Dinv + (st & 1) * nd),
+                                   Dinv + ((st + 1) & 1) * nd, (const double *)odiag, dead);
+                continue;
+            }
+            diag(st, Ain);
+            hipLaunchKernelGGL(k_gj_panel, dim3(blocks_for((int64_t)nbmax * 4, 256), G), dim3(256), 0, c->stream, st * GJ_NB,
+                               (const int32_t *)c->cgrp_cb, (const int64_t *)c->cgrp_off, Ain, (const double *)Dinv, Rt);
+            hipLaunchKernelGGL(k_gj_update, dim3(T * T, G), dim3(256), 0, c->stream, st * GJ_NB, T, (const int32_t *)c->cgrp_cb,
+                               (const int64_t *)c->cgrp_off, Ain, Aout, (const double *)Dinv, (const double *)Rt);
         }
         hipLaunchKernelGGL(k_coarse_undead, gsq, dim3(256), 0, c->stream, (const int32_t *)c->cgrp_cb,
                            (const int64_t *)c->cgrp_off, (nsteps & 1) ? A1 : A0, (const uint8_t *)dead);

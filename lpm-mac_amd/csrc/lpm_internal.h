@@ -147,6 +147,7 @@ struct lpm_ctx {
     double *agg_d = nullptr;          // x0_i - centre of its aggregate (dim entries per particle)
     int32_t *ra_row = nullptr, *ra_id = nullptr;  // distinct aggregates of the columns of each row: row, aggregate
     int64_t nra = 0;
+    bool gj_fused = false;            // the inversion's steps as one launch each (GJ_FUSED_TILES in kernels_coarse.hip)
     int32_t *cq_ptr = nullptr, *cq_f = nullptr, *cq_gh = nullptr;  // coarse blocks: contributing row entries
     int64_t ncq = 0;
     double *cvbuf = nullptr;          // per (row, aggregate) contributions P_i^T K_ij P_j (nmode^2 each)
