@@ -191,7 +191,9 @@ int64_t lpm_size(const lpm_ctx *ctx, const char *what);
  *                        kept under cg_graph, spmv_tune = 0 (the caller fixes the SpMV launch) and
  *                        per-SpMV timing. lpm_stat("cg_persistent") counts the persistent solves
  *  "cg_wait_ms"       longest wait between workgroups inside a persistent solve (0..60000, default
- *                        2000); a solve that exceeds it is repeated with launches
+ *                        2000); a solve that exceeds it is repeated with launches, and later solves
+ *                        of the context are launched at once until cg_wait_ms or cg_persist is set
+ *                        again. lpm_stat("cg_persist_given_up") counts such solves
  *  "cg_batch"         CG iterations issued before the host reads the device's stop flag (rounded
  *                        up to even; default 16); iterations issued past the stop are no-ops, so
  *                        the batch sizes never change results

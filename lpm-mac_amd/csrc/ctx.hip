@@ -1042,10 +1042,14 @@ int lpm_set_mode(lpm_ctx *c, const char *name, double v) {
     else if (w == "cg_forcing") c->cg_forcing = (int)v ? 1 : 0;
     else if (w == "coarse_graph") c->coarse_graph = (int)v ? 1 : 0;
     else if (w == "cg_graph") c->cg_graph = (int)v ? 1 : 0;
-    else if (w == "cg_persist") c->cg_persist = (int)v ? 1 : 0;
+    else if (w == "cg_persist") {
+        c->cg_persist = (int)v ? 1 : 0;
+        c->pcg_given_up = false;
+    }
     else if (w == "cg_wait_ms") {
         if (!(v >= 0 && v <= 60000)) return lpm_fail(c, LPM_E_ARG, "cg_wait_ms must be 0..60000");
         c->cg_wait_ms = v;
+        c->pcg_given_up = false;
     }
     else if (w == "coarse_reuse") c->coarse_reuse = (int)v ? 1 : 0;
     else if (w == "coarse_rebuild") {
@@ -1402,6 +1406,7 @@ double lpm_stat(const lpm_ctx *c, const char *name) {
     if (w == "coarse_builds") return (double)c->st_coarse_builds;
     if (w == "cg_solves") return (double)c->st_cg_solves;
     if (w == "cg_persistent") return (double)c->st_pcg;
+    if (w == "cg_persist_given_up") return (double)c->st_pcg_given_up;
     if (w == "assemblies") return (double)c->st_asm;
     if (w == "spmv_launches") return (double)c->st_spmv;
     if (w == "spmv_ms") return c->st_spmv_ms;
@@ -1416,7 +1421,7 @@ double lpm_stat(const lpm_ctx *c, const char *name) {
 int lpm_reset_stats(lpm_ctx *c) {
     if (!c) return LPM_E_ARG;
     c->st_newton = c->st_cg_iters = c->st_cg_solves = c->st_asm = c->st_spmv = c->st_spmv_timed = 0;
-    c->st_coarse_builds = c->st_pcg = 0;
+    c->st_coarse_builds = c->st_pcg = c->st_pcg_given_up = 0;
     c->st_spmv_ms = 0;
     return LPM_OK;
 }

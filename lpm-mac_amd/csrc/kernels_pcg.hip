@@ -41,7 +41,8 @@
 //
 // The grid has at most one workgroup per CU and is launched cooperatively, so all of it is resident.
 // Every wait is bounded all the same: a workgroup that has polled for cg_wait_ms sets SC_ABORT and
-// leaves, the others see it and leave, and the host solves the system again launch by launch.
+// leaves, the others see it and leave, and the host solves the system again launch by launch, as it does all
+// later ones of the context until cg_persist or cg_wait_ms is set again.
 #include <algorithm>
 #include <cfloat>
 #include <vector>
@@ -669,7 +670,11 @@ static int pcg_go(lpm_ctx *c, PcgArgs &a, int64_t maxit, bool *ran) {
         }
         LPM_HIP(c, hipMemcpyAsync(c->h_scal, c->scal, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, c->stream));
         LPM_HIP(c, hipStreamSynchronize(c->stream));
-        if (c->h_scal[SC_ABORT] != 0.0) return LPM_OK;
+        if (c->h_scal[SC_ABORT] != 0.0) {  // what holds the device may hold it for long: no further wait in this context
+            c->pcg_given_up = true;
+            c->st_pcg_given_up++;
+            return LPM_OK;
+        }
         if (c->h_scal[SC_DONE] != 0.0) {
             *ran = true;
             return LPM_OK;
@@ -685,7 +690,7 @@ int pcg_solve(lpm_ctx *c, int64_t maxit, bool *ran) {
     *ran = false;
     // a caller that fixes the SpMV launch shape, replays batches from a graph or times single SpMVs
     // asks for the launches themselves
-    if (!c->cg_persist || c->cg_graph || !c->spmv_tune || c->timing > 0) return LPM_OK;
+    if (!c->cg_persist || c->cg_graph || !c->spmv_tune || c->timing > 0 || c->pcg_given_up) return LPM_OK;
     int rc = pcg_prepare(c);
     if (rc || c->pcg_state != 1) return rc;
     PcgArgs a = {};

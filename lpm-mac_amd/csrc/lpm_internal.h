@@ -174,7 +174,8 @@ struct lpm_ctx {
     double cg_wait_ms = 2000;         // longest wait inside the kernel before the solve is done by launches
     int pcg_state = 0, pcg_coarse = 0;  // 0 not prepared, 1 usable, -1 not; whether it has the coarse lists
     int pcg_spw = 0, pcg_grid = 0, pcg_nslot_c = 0, pcg_nl = 0;  // pcg_nl: most aggregates of a workgroup
-    int64_t pcg_words = 0, st_pcg = 0;  // st_pcg: solves it did
+    int64_t pcg_words = 0, st_pcg = 0, st_pcg_given_up = 0;  // solves it did, and gave up
+    bool pcg_given_up = false;        // after one given up: launches until cg_persist or cg_wait_ms is set
     void *pcg_slots = nullptr;
     const void *pcg_kern = nullptr;   // the kernel and LDS size the next two were found for
     size_t pcg_lds = 0;
