@@ -189,7 +189,9 @@ int64_t lpm_size(const lpm_ctx *ctx, const char *what);
  *                        persistent launch (the same recurrence, stopping rule and precision) |
  *                        0: one launch per step of every iteration. Launched solves are also
  *                        kept under cg_graph, spmv_tune = 0 (the caller fixes the SpMV launch) and
- *                        per-SpMV timing. lpm_stat("cg_persistent") counts the persistent solves
+ *                        per-SpMV timing. lpm_stat("cg_persistent") counts the persistent solves,
+ *                        lpm_stat("cg_persist_plans") how often a context prepared for them (once
+ *                        with and once without the coarse space)
  *  "cg_wait_ms"       longest wait between workgroups inside a persistent solve (0..60000, default
  *                        2000); a solve that exceeds it is repeated with launches, and later solves
  *                        of the context are launched at once until cg_wait_ms or cg_persist is set

@@ -1406,6 +1406,7 @@ double lpm_stat(const lpm_ctx *c, const char *name) {
     if (w == "coarse_builds") return (double)c->st_coarse_builds;
     if (w == "cg_solves") return (double)c->st_cg_solves;
     if (w == "cg_persistent") return (double)c->st_pcg;
+    if (w == "cg_persist_plans") return (double)c->st_pcg_plans;
     if (w == "cg_persist_given_up") return (double)c->st_pcg_given_up;
     if (w == "assemblies") return (double)c->st_asm;
     if (w == "spmv_launches") return (double)c->st_spmv;

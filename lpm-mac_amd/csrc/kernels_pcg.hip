@@ -538,25 +538,22 @@ __global__ __launch_bounds__(256) void k_pcg_clear(int64_t words, u64 *slots, do
 // workgroup that forms any polls all shares of its group
 static int dofs_per_wg(int ncoarse, int G) { return std::max(PCG_NW, (ncoarse + G - 1) / G); }
 
-// Slots and, for the two-level preconditioner, the rows of each workgroup by aggregate. Built once
-// for a pattern, again when the coarse space appears. Sets c->pcg_state: 1 usable, -1 not.
-static int pcg_prepare(lpm_ctx *c) {
-    const int coarse = two_level(c) ? 1 : 0;
-    if (c->pcg_state != 0 && c->pcg_coarse == coarse) return LPM_OK;
-    pcg_free(c);
-    c->pcg_coarse = coarse;
-    c->pcg_state = -1;
+// Slots and, for the two-level preconditioner, the rows of each workgroup by aggregate: built once for each of
+// the two kinds and kept, since a caller may switch between them from solve to solve (SC 40^3: 0.5 ms a time).
+// Sets the plan's state: 1 usable, -1 not.
+static int pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
+    if (P.state != 0) return LPM_OK;
+    P.state = -1;
     const int spw = (int)((c->nslice + PCG_WG - 1) / PCG_WG);
     if (spw > PCG_SPW) return LPM_OK;  // more than one row per thread
     const int G = (int)((c->nslice + spw - 1) / spw), D = c->dim, M = D == 3 ? 6 : 3;
     // 32-bit buffer offsets, FP64 values at most
     if ((double)c->nslots * D * D * 8 > 4.0e9) return LPM_OK;
     int64_t nctr = 0;
-    c->pcg_nl = 0;
     // Slices in id order, or, with the coarse space, by the aggregate of their middle row: slices that
     // lie side by side across the numbering direction then meet in one workgroup, which so
     // touches fewer aggregates (hex 200 x 231: 6 instead of 15).
-    std::vector<int32_t> order(c->nslice);
+    std::vector<int32_t> order(c->nslice), lptr(1, 0), lagg, slot, lbeg, wpos, cnt;
     for (int64_t k = 0; k < c->nslice; ++k) order[k] = (int32_t)k;
     if (coarse) {
         const int64_t n = c->n;
@@ -569,7 +566,8 @@ static int pcg_prepare(lpm_ctx *c) {
             std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
                 return agg[std::min<int64_t>(n - 1, 64LL * x + 32)] < agg[std::min<int64_t>(n - 1, 64LL * y + 32)];
             });
-        std::vector<int32_t> lptr(1, 0), lagg, lbeg, wpos(n), rank(c->nagg, -1), fill;
+        std::vector<int32_t> rank(c->nagg, -1), fill;
+        wpos.resize(n);
         for (int w = 0; w < G; ++w) {
             std::vector<int64_t> rows;
             for (int64_t q = (int64_t)w * spw; q < std::min<int64_t>(c->nslice, (int64_t)(w + 1) * spw); ++q)
@@ -589,50 +587,47 @@ static int pcg_prepare(lpm_ctx *c) {
                 wpos[i] = (q << 16) | fill[q]++;
             }
             lagg.insert(lagg.end(), mine.begin(), mine.end());
-            c->pcg_nl = std::max(c->pcg_nl, (int)mine.size());
             lptr.push_back((int32_t)lagg.size());
         }
         const int per = dofs_per_wg(c->ncoarse, G);
         for (int y = 0; y < c->ncoarse; y += per)
             if (cb[grp[(std::min(c->ncoarse, y + per) - 1) / M] + 1] - cb[grp[y / M]] > PCG_CZ) return LPM_OK;
         // share u of coarse DoF d lies at u * ncoarse + d, so that a wavefront's polls are contiguous
-        std::vector<int32_t> cnt(c->nagg, 0), slot(lagg.size());
+        cnt.assign(c->nagg, 0);
+        slot.resize(lagg.size());
         for (size_t q = 0; q < lagg.size(); ++q) slot[q] = cnt[lagg[q]]++;
         nctr = (int64_t)*std::max_element(cnt.begin(), cnt.end()) * c->ncoarse;
-        const std::vector<int32_t> *all[6] = {&lptr, &lagg, &slot, &lbeg, &wpos, &cnt};
-        int32_t **dst[6] = {&c->pcg_lptr, &c->pcg_lagg, &c->pcg_lslot, &c->pcg_lbeg, &c->pcg_wpos, &c->pcg_cnt};
-        for (int k = 0; k < 6; ++k) {
-            LPM_HIP(c, hipMalloc(dst[k], sizeof(int32_t) * all[k]->size()));
-            LPM_HIP(c, hipMemcpyAsync(*dst[k], all[k]->data(), sizeof(int32_t) * all[k]->size(), hipMemcpyHostToDevice, c->stream));
-        }
-        LPM_HIP(c, hipStreamSynchronize(c->stream));
     }
-    LPM_HIP(c, hipMalloc(&c->pcg_order, sizeof(int32_t) * c->nslice));
-    LPM_HIP(c, hipMemcpyAsync(c->pcg_order, order.data(), sizeof(int32_t) * c->nslice, hipMemcpyHostToDevice, c->stream));
+    P.words = 2 * (nctr + (coarse ? c->ncoarse : 0) + 3 * (int64_t)PCG_SET);
+    P.nslot_c = (int)nctr;
+    Slab slab;
+    slab.add(&P.slots, P.words);
+    const std::vector<int32_t> *src[7] = {&order, &lptr, &lagg, &slot, &lbeg, &wpos, &cnt};
+    int32_t **dst[7] = {&P.order, &P.lptr, &P.lagg, &P.lslot, &P.lbeg, &P.wpos, &P.cnt};
+    for (int k = 0; k < 7; ++k) slab.add(dst[k], (int64_t)src[k]->size());
+    LPM_HIP(c, slab.alloc(&P.base));
+    for (int k = 0; k < 7; ++k)
+        if (!src[k]->empty())
+            LPM_HIP(c, hipMemcpyAsync(*dst[k], src[k]->data(), sizeof(int32_t) * src[k]->size(), hipMemcpyHostToDevice, c->stream));
     LPM_HIP(c, hipStreamSynchronize(c->stream));
-    c->pcg_words = 2 * (nctr + (coarse ? c->ncoarse : 0) + 3 * (int64_t)PCG_SET);
-    c->pcg_nslot_c = (int)nctr;
-    LPM_HIP(c, hipMalloc(&c->pcg_slots, sizeof(u64) * c->pcg_words));
-    c->pcg_spw = spw;
-    c->pcg_grid = G;
-    c->pcg_state = 1;
+    P.spw = spw;
+    P.grid = G;
+    P.state = 1;
+    c->st_pcg_plans++;
     return LPM_OK;
 }
 
 void pcg_free(lpm_ctx *c) {
-    for (void *p : {(void *)c->pcg_lptr, (void *)c->pcg_lagg, (void *)c->pcg_lslot, (void *)c->pcg_lbeg, (void *)c->pcg_wpos,
-                    (void *)c->pcg_cnt, (void *)c->pcg_slots, (void *)c->pcg_order})
-        if (p) hipFree(p);
-    c->pcg_lptr = c->pcg_lagg = c->pcg_lslot = c->pcg_lbeg = c->pcg_wpos = c->pcg_cnt = c->pcg_order = nullptr;
-    c->pcg_slots = nullptr;
-    c->pcg_kern = nullptr;
-    c->pcg_state = 0;
+    for (PcgPlan &P : c->pcg_plan) {
+        if (P.base) hipFree(P.base);
+        P = PcgPlan();
+    }
 }
 
 template <typename T, int D, typename IX, bool NT>
-static int pcg_go(lpm_ctx *c, PcgArgs &a, int64_t maxit, bool *ran) {
+static int pcg_go(lpm_ctx *c, PcgPlan &P, PcgArgs &a, int64_t maxit, bool *ran) {
     const int M = D == 3 ? 6 : 3;
-    const size_t un = std::max(sizeof(T) * PCG_NW * D * 64, sizeof(double) * M * 64 * (size_t)c->pcg_spw);
+    const size_t un = std::max(sizeof(T) * PCG_NW * D * 64, sizeof(double) * M * 64 * (size_t)P.spw);
     size_t lds = un + sizeof(double) * (PCG_CZ + PCG_LA * M);
     // a workgroup's rows of Ac^-1 stay in its LDS where they fit beside the rest
     a.ainv_lds = 0;
@@ -642,26 +637,26 @@ static int pcg_go(lpm_ctx *c, PcgArgs &a, int64_t maxit, bool *ran) {
         lds += rows;
     }
     auto kern = k_pcg<T, D, IX, NT>;
-    if (c->pcg_kern != (const void *)kern || c->pcg_lds != lds) {  // all workgroups must be resident at once
+    if (P.kern != (const void *)kern || P.lds != lds) {  // all workgroups must be resident at once
         int per = 0, cus = 0, khz = 0;
         LPM_HIP(c, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         LPM_HIP(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, PCG_NT, lds));
         LPM_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
         LPM_HIP(c, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device));
-        c->pcg_kern = (const void *)kern;
-        c->pcg_lds = lds;
-        c->pcg_fits = (int64_t)per * cus >= c->pcg_grid;
-        c->pcg_khz = khz;
+        P.kern = (const void *)kern;
+        P.lds = lds;
+        P.fits = (int64_t)per * cus >= P.grid;
+        P.khz = khz;
     }
-    if (!c->pcg_fits) return LPM_OK;
-    a.wait_ticks = (u64)(c->cg_wait_ms * c->pcg_khz);
+    if (!P.fits) return LPM_OK;
+    a.wait_ticks = (u64)(c->cg_wait_ms * P.khz);
     for (int64_t it = 0;;) {
-        hipLaunchKernelGGL(k_pcg_clear, dim3(blocks_for(c->pcg_words, 256)), dim3(256), 0, c->stream, c->pcg_words,
-                           (u64 *)c->pcg_slots, c->scal);
+        hipLaunchKernelGGL(k_pcg_clear, dim3(blocks_for(P.words, 256)), dim3(256), 0, c->stream, P.words,
+                           P.slots, c->scal);
         a.it0 = (int)it;
         a.itmax = (int)std::min<int64_t>(it + PCG_LAUNCH_ITERS, 0x7fffffff);
         void *args[] = {&a};
-        const hipError_t e = hipLaunchCooperativeKernel((const void *)kern, dim3(c->pcg_grid), dim3(PCG_NT), args, (unsigned)lds,
+        const hipError_t e = hipLaunchCooperativeKernel((const void *)kern, dim3(P.grid), dim3(PCG_NT), args, (unsigned)lds,
                                                         c->stream);
         if (e != hipSuccess) {
             if (it > 0) return lpm_fail(c, LPM_E_HIP, std::string("k_pcg: ") + hipGetErrorString(e));
@@ -691,16 +686,17 @@ int pcg_solve(lpm_ctx *c, int64_t maxit, bool *ran) {
     // a caller that fixes the SpMV launch shape, replays batches from a graph or times single SpMVs
     // asks for the launches themselves
     if (!c->cg_persist || c->cg_graph || !c->spmv_tune || c->timing > 0 || c->pcg_given_up) return LPM_OK;
-    int rc = pcg_prepare(c);
-    if (rc || c->pcg_state != 1) return rc;
-    PcgArgs a = {};
     const bool coarse = two_level(c);
+    PcgPlan &P = c->pcg_plan[coarse ? 1 : 0];
+    int rc = pcg_prepare(c, P, coarse);
+    if (rc || P.state != 1) return rc;
+    PcgArgs a = {};
     const size_t es = c->precision == 0 ? 4 : 8;
     const int D = c->dim;
     const bool idx16 = c->scol16 && c->spmv_idx16;
     a.n = c->n;
     a.nslice = c->nslice;
-    a.spw = c->pcg_spw;
+    a.spw = P.spw;
     a.block_pre = block_jacobi(c);
     a.coarse = coarse;
     a.tol = c->cg_tol;
@@ -720,30 +716,30 @@ int pcg_solve(lpm_ctx *c, int64_t maxit, bool *ran) {
     a.p = c->v_p;
     a.s = c->v_s;
     a.scal = c->scal;
-    u64 *w = (u64 *)c->pcg_slots;
+    u64 *w = P.slots;
     a.slot_u = w;
     a.slot_d = w + 4 * PCG_SET;
     a.slot_c = w + 6 * PCG_SET;
-    a.nslot_c = c->pcg_nslot_c;
+    a.nslot_c = P.nslot_c;
     a.slot_y = a.slot_c + 2 * (int64_t)a.nslot_c;
     a.ncoarse = coarse ? c->ncoarse : 0;
-    a.ndof_wg = dofs_per_wg(a.ncoarse, c->pcg_grid);
+    a.ndof_wg = dofs_per_wg(a.ncoarse, P.grid);
     a.agg_d = c->agg_d;
     a.Ainv = c->Ainv;
     a.mask = c->dofmask;
     a.agg_grp = c->agg_grp;
     a.cb = c->cgrp_cb;
     a.off = c->cgrp_off;
-    a.ca_cnt = c->pcg_cnt;
-    a.wl_ptr = c->pcg_lptr;
-    a.wl_agg = c->pcg_lagg;
-    a.wl_slot = c->pcg_lslot;
-    a.wl_beg = c->pcg_lbeg;
-    a.wpos = c->pcg_wpos;
-    a.order = c->pcg_order;
+    a.ca_cnt = P.cnt;
+    a.wl_ptr = P.lptr;
+    a.wl_agg = P.lagg;
+    a.wl_slot = P.lslot;
+    a.wl_beg = P.lbeg;
+    a.wpos = P.wpos;
+    a.order = P.order;
     // the matrix is kept in the L2s while it fits them (8 x 4 MB) and streamed past them otherwise
     const bool nt = (double)c->nslots * (D * D * es + (idx16 ? 2 : 4)) > 28e6 && c->spmv_nt;
-#define PCG_GO(T, D_, IX) (nt ? pcg_go<T, D_, IX, true>(c, a, maxit, ran) : pcg_go<T, D_, IX, false>(c, a, maxit, ran))
+#define PCG_GO(T, D_, IX) (nt ? pcg_go<T, D_, IX, true>(c, P, a, maxit, ran) : pcg_go<T, D_, IX, false>(c, P, a, maxit, ran))
     if (c->precision == 0) {
         if (D == 3) return idx16 ? PCG_GO(float, 3, int16_t) : PCG_GO(float, 3, int32_t);
         return idx16 ? PCG_GO(float, 2, int16_t) : PCG_GO(float, 2, int32_t);

@@ -82,6 +82,20 @@ struct Slab {
     }
 };
 
+// The persistent CG's workgroups and what they exchange (kernels_pcg.hip), for one kind of preconditioner
+struct PcgPlan {
+    int state = 0;                        // 0 not prepared, 1 usable, -1 not
+    int spw = 0, grid = 0, nslot_c = 0;   // slices of a workgroup, workgroups, words of one set of coarse shares
+    int64_t words = 0;                    // of all slots
+    void *base = nullptr;                 // the one allocation that holds the arrays below
+    unsigned long long *slots = nullptr;
+    int32_t *lptr = nullptr, *lagg = nullptr, *lslot = nullptr, *lbeg = nullptr, *wpos = nullptr, *cnt = nullptr, *order = nullptr;
+    const void *kern = nullptr;           // the kernel and LDS size that `fits` was found for
+    size_t lds = 0;
+    bool fits = false;                    // its whole grid can be resident
+    int khz = 0;                          // rate of the device's wall clock
+};
+
 struct lpm_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -172,17 +186,9 @@ struct lpm_ctx {
     // slots they exchange partial sums in, and each workgroup's rows by aggregate
     int cg_persist = 1;
     double cg_wait_ms = 2000;         // longest wait inside the kernel before the solve is done by launches
-    int pcg_state = 0, pcg_coarse = 0;  // 0 not prepared, 1 usable, -1 not; whether it has the coarse lists
-    int pcg_spw = 0, pcg_grid = 0, pcg_nslot_c = 0, pcg_nl = 0;  // pcg_nl: most aggregates of a workgroup
-    int64_t pcg_words = 0, st_pcg = 0, st_pcg_given_up = 0;  // solves it did, and gave up
+    int64_t st_pcg = 0, st_pcg_given_up = 0, st_pcg_plans = 0;  // solves it did, and gave up; plans built
     bool pcg_given_up = false;        // after one given up: launches until cg_persist or cg_wait_ms is set
-    void *pcg_slots = nullptr;
-    const void *pcg_kern = nullptr;   // the kernel and LDS size the next two were found for
-    size_t pcg_lds = 0;
-    bool pcg_fits = false;            // its whole grid can be resident
-    int pcg_khz = 0;                  // rate of the device's wall clock
-    int32_t *pcg_lptr = nullptr, *pcg_lagg = nullptr, *pcg_lslot = nullptr, *pcg_lbeg = nullptr, *pcg_wpos = nullptr,
-            *pcg_cnt = nullptr, *pcg_order = nullptr;
+    PcgPlan pcg_plan[2];              // without and with the coarse space
     int coarse_graph = 0;             // 1: replay the inversion from a HIP graph, 0: launch directly
     // Load-step predictor (mode "predictor"): free DoFs start each step from the converged
     // position extrapolated from the previous converged steps: 1 linearly (plus the previous
