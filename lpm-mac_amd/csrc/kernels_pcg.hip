@@ -538,17 +538,23 @@ __global__ __launch_bounds__(256) void k_pcg_clear(int64_t words, u64 *slots, do
 // workgroup that forms any polls all shares of its group
 static int dofs_per_wg(int ncoarse, int G) { return std::max(PCG_NW, (ncoarse + G - 1) / G); }
 
+// whether a runtime call succeeded; the error of one that did not is cleared, since the launches take over
+static bool hip_done(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
 // Slots and, for the two-level preconditioner, the rows of each workgroup by aggregate: built once for each of
 // the two kinds and kept, since a caller may switch between them from solve to solve (SC 40^3: 0.5 ms a time).
-// Sets the plan's state: 1 usable, -1 not.
-static int pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
-    if (P.state != 0) return LPM_OK;
+// Sets the plan's state: 1 usable, -1 not. No failure in here ends the solve: the launches need none of this.
+static void pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
+    if (P.state != 0) return;
     P.state = -1;
     const int spw = (int)((c->nslice + PCG_WG - 1) / PCG_WG);
-    if (spw > PCG_SPW) return LPM_OK;  // more than one row per thread
+    if (spw > PCG_SPW) return;  // more than one row per thread
     const int G = (int)((c->nslice + spw - 1) / spw), D = c->dim, M = D == 3 ? 6 : 3;
     // 32-bit buffer offsets, FP64 values at most
-    if ((double)c->nslots * D * D * 8 > 4.0e9) return LPM_OK;
+    if ((double)c->nslots * D * D * 8 > 4.0e9) return;
     int64_t nctr = 0;
     // Slices in id order, or, with the coarse space, by the aggregate of their middle row: slices that
     // lie side by side across the numbering direction then meet in one workgroup, which so
@@ -558,10 +564,11 @@ static int pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
     if (coarse) {
         const int64_t n = c->n;
         std::vector<int32_t> agg(n), grp(c->nagg), cb(c->ncgrp + 1);
-        LPM_HIP(c, hipMemcpyAsync(agg.data(), c->agg_of, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream));
-        LPM_HIP(c, hipMemcpyAsync(grp.data(), c->agg_grp, sizeof(int32_t) * c->nagg, hipMemcpyDeviceToHost, c->stream));
-        LPM_HIP(c, hipMemcpyAsync(cb.data(), c->cgrp_cb, sizeof(int32_t) * (c->ncgrp + 1), hipMemcpyDeviceToHost, c->stream));
-        LPM_HIP(c, hipStreamSynchronize(c->stream));
+        if (!hip_done(hipMemcpyAsync(agg.data(), c->agg_of, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream)) ||
+            !hip_done(hipMemcpyAsync(grp.data(), c->agg_grp, sizeof(int32_t) * c->nagg, hipMemcpyDeviceToHost, c->stream)) ||
+            !hip_done(hipMemcpyAsync(cb.data(), c->cgrp_cb, sizeof(int32_t) * (c->ncgrp + 1), hipMemcpyDeviceToHost, c->stream)) ||
+            !hip_done(hipStreamSynchronize(c->stream)))
+            return;
         if (spw > 1)
             std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
                 return agg[std::min<int64_t>(n - 1, 64LL * x + 32)] < agg[std::min<int64_t>(n - 1, 64LL * y + 32)];
@@ -576,7 +583,7 @@ static int pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
             for (int64_t i : rows) mine.push_back(agg[i]);
             std::sort(mine.begin(), mine.end());
             mine.erase(std::unique(mine.begin(), mine.end()), mine.end());
-            if ((int)mine.size() > PCG_LA) return LPM_OK;
+            if ((int)mine.size() > PCG_LA) return;
             fill.assign(mine.size() + 1, 0);
             for (size_t q = 0; q < mine.size(); ++q) rank[mine[q]] = (int32_t)q;
             for (int64_t i : rows) ++fill[rank[agg[i]] + 1];
@@ -591,7 +598,7 @@ static int pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
         }
         const int per = dofs_per_wg(c->ncoarse, G);
         for (int y = 0; y < c->ncoarse; y += per)
-            if (cb[grp[(std::min(c->ncoarse, y + per) - 1) / M] + 1] - cb[grp[y / M]] > PCG_CZ) return LPM_OK;
+            if (cb[grp[(std::min(c->ncoarse, y + per) - 1) / M] + 1] - cb[grp[y / M]] > PCG_CZ) return;
         // share u of coarse DoF d lies at u * ncoarse + d, so that a wavefront's polls are contiguous
         cnt.assign(c->nagg, 0);
         slot.resize(lagg.size());
@@ -605,16 +612,16 @@ static int pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
     const std::vector<int32_t> *src[7] = {&order, &lptr, &lagg, &slot, &lbeg, &wpos, &cnt};
     int32_t **dst[7] = {&P.order, &P.lptr, &P.lagg, &P.lslot, &P.lbeg, &P.wpos, &P.cnt};
     for (int k = 0; k < 7; ++k) slab.add(dst[k], (int64_t)src[k]->size());
-    LPM_HIP(c, slab.alloc(&P.base));
+    if (!hip_done(slab.alloc(&P.base))) return;
     for (int k = 0; k < 7; ++k)
-        if (!src[k]->empty())
-            LPM_HIP(c, hipMemcpyAsync(*dst[k], src[k]->data(), sizeof(int32_t) * src[k]->size(), hipMemcpyHostToDevice, c->stream));
-    LPM_HIP(c, hipStreamSynchronize(c->stream));
+        if (!src[k]->empty() && !hip_done(hipMemcpyAsync(*dst[k], src[k]->data(), sizeof(int32_t) * src[k]->size(),
+                                                         hipMemcpyHostToDevice, c->stream)))
+            return;
+    if (!hip_done(hipStreamSynchronize(c->stream))) return;
     P.spw = spw;
     P.grid = G;
     P.state = 1;
     c->st_pcg_plans++;
-    return LPM_OK;
 }
 
 void pcg_free(lpm_ctx *c) {
@@ -629,23 +636,35 @@ static int pcg_go(lpm_ctx *c, PcgPlan &P, PcgArgs &a, int64_t maxit, bool *ran) 
     const int M = D == 3 ? 6 : 3;
     const size_t un = std::max(sizeof(T) * PCG_NW * D * 64, sizeof(double) * M * 64 * (size_t)P.spw);
     size_t lds = un + sizeof(double) * (PCG_CZ + PCG_LA * M);
+    auto kern = k_pcg<T, D, IX, NT>;
+    if (P.kern != (const void *)kern) {
+        // The device's LDS less the kernel's own. Every context asks for this same limit, as the attribute belongs
+        // to the kernel and not to the context.
+        hipFuncAttributes fa;
+        int most = 0;
+        P.kern = (const void *)kern;
+        P.lds = 0;
+        P.lds_most = 0;
+        if (hip_done(hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device)) &&
+            hip_done(hipFuncGetAttributes(&fa, (const void *)kern)) && (size_t)most > fa.sharedSizeBytes &&
+            hip_done(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, most - (int)fa.sharedSizeBytes)))
+            P.lds_most = most - fa.sharedSizeBytes;
+    }
+    if (lds > P.lds_most) return LPM_OK;
     // a workgroup's rows of Ac^-1 stay in its LDS where they fit beside the rest
     a.ainv_lds = 0;
     const size_t rows = sizeof(double) * (size_t)a.ndof_wg * std::max(c->cgrp_nbmax, 1);
-    if (a.coarse && lds + rows <= 150 * 1024) {
+    if (a.coarse && lds + rows <= P.lds_most) {
         a.ainv_lds = c->cgrp_nbmax;
         lds += rows;
     }
-    auto kern = k_pcg<T, D, IX, NT>;
-    if (P.kern != (const void *)kern || P.lds != lds) {  // all workgroups must be resident at once
+    if (P.lds != lds) {  // all workgroups must be resident at once
         int per = 0, cus = 0, khz = 0;
-        LPM_HIP(c, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        LPM_HIP(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, PCG_NT, lds));
-        LPM_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-        LPM_HIP(c, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device));
-        P.kern = (const void *)kern;
+        P.fits = hip_done(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, PCG_NT, lds)) &&
+                 hip_done(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device)) &&
+                 hip_done(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device)) &&
+                 (int64_t)per * cus >= P.grid;
         P.lds = lds;
-        P.fits = (int64_t)per * cus >= P.grid;
         P.khz = khz;
     }
     if (!P.fits) return LPM_OK;
@@ -658,9 +677,8 @@ static int pcg_go(lpm_ctx *c, PcgPlan &P, PcgArgs &a, int64_t maxit, bool *ran) 
         void *args[] = {&a};
         const hipError_t e = hipLaunchCooperativeKernel((const void *)kern, dim3(P.grid), dim3(PCG_NT), args, (unsigned)lds,
                                                         c->stream);
-        if (e != hipSuccess) {
-            if (it > 0) return lpm_fail(c, LPM_E_HIP, std::string("k_pcg: ") + hipGetErrorString(e));
-            (void)hipGetLastError();  // no cooperative launch here: the caller solves launch by launch
+        if (!hip_done(e)) {  // no cooperative launch here: the caller solves launch by launch
+            P.fits = false;
             return LPM_OK;
         }
         LPM_HIP(c, hipMemcpyAsync(c->h_scal, c->scal, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, c->stream));
@@ -688,8 +706,8 @@ int pcg_solve(lpm_ctx *c, int64_t maxit, bool *ran) {
     if (!c->cg_persist || c->cg_graph || !c->spmv_tune || c->timing > 0 || c->pcg_given_up) return LPM_OK;
     const bool coarse = two_level(c);
     PcgPlan &P = c->pcg_plan[coarse ? 1 : 0];
-    int rc = pcg_prepare(c, P, coarse);
-    if (rc || P.state != 1) return rc;
+    pcg_prepare(c, P, coarse);
+    if (P.state != 1) return LPM_OK;
     PcgArgs a = {};
     const size_t es = c->precision == 0 ? 4 : 8;
     const int D = c->dim;

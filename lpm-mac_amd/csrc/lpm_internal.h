@@ -90,8 +90,8 @@ struct PcgPlan {
     void *base = nullptr;                 // the one allocation that holds the arrays below
     unsigned long long *slots = nullptr;
     int32_t *lptr = nullptr, *lagg = nullptr, *lslot = nullptr, *lbeg = nullptr, *wpos = nullptr, *cnt = nullptr, *order = nullptr;
-    const void *kern = nullptr;           // the kernel and LDS size that `fits` was found for
-    size_t lds = 0;
+    const void *kern = nullptr;           // the kernel, the most LDS it may ask for, the LDS that `fits` was found for
+    size_t lds_most = 0, lds = 0;
     bool fits = false;                    // its whole grid can be resident
     int khz = 0;                          // rate of the device's wall clock
 };
