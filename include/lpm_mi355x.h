@@ -191,7 +191,11 @@ int64_t lpm_size(const lpm_ctx *ctx, const char *what);
  *                        kept under cg_graph, spmv_tune = 0 (the caller fixes the SpMV launch) and
  *                        per-SpMV timing. lpm_stat("cg_persistent") counts the persistent solves,
  *                        lpm_stat("cg_persist_plans") how often a context prepared for them (once
- *                        with and once without the coarse space)
+ *                        with and once without the coarse space). Contexts that solve at the same
+ *                        time from several threads share the CUs out: small systems run side by
+ *                        side, systems of more than 16,384 particles mostly one after the other,
+ *                        for which 0 can give more throughput (four of 64,000: 30 against 41 us
+ *                        per iteration)
  *  "cg_wait_ms"       longest wait between workgroups inside a persistent solve (0..60000, default
  *                        2000); a solve that exceeds it is repeated with launches, and later solves
  *                        of the context are launched at once until cg_wait_ms or cg_persist is set

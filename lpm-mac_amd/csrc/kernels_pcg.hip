@@ -39,12 +39,19 @@
 // 256 registers hold a row's state and eight slots in flight; with sixteen of 128 the compiler spilled
 // 70-150 registers and the kernel lost to the launches (hex 200 x 231: 31.9-42.6 us).
 //
-// The grid has at most one workgroup per CU and is launched cooperatively, so all of it is resident.
+// The grid has at most one workgroup per CU, so all of it is resident: the solves that contexts run at the same time
+// from several threads share the CUs out (ResidentCus), and other kernels end. Cooperative launches give the
+// same promise, but run one after the other on the device. us per iteration over all of four contexts in threads
+// of their own, launch by launch, cooperative, and with the CUs shared out: SC 12^3 8.3, 15.3, 4.0; hex 60 x 60 6.9,
+// 12.4, 3.2; SC 20^3 10.5, 17.7, 9.8; SC 40^3, whose grid takes every CU, 29.7, 40.4, 40.9 (one context: 47.2, 40.4, 40.3).
 // Every wait is bounded all the same: a workgroup that has polled for cg_wait_ms sets SC_ABORT and
 // leaves, the others see it and leave, and the host solves the system again launch by launch, as it does all
 // later ones of the context until cg_persist or cg_wait_ms is set again.
 #include <algorithm>
 #include <cfloat>
+#include <condition_variable>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "lpm_internal.h"
@@ -631,6 +638,49 @@ void pcg_free(lpm_ctx *c) {
     }
 }
 
+namespace {
+
+// The CUs of each device, dealt out to the persistent solves in flight, in the order in which they ask. Workgroups
+// go round the eight XCDs, so a grid takes ceil(grid / 8) CUs of each.
+class ResidentCus {
+public:
+    ResidentCus(int device, int cus, int grid) : d_(of(device)) {
+        const int all = std::max(1, cus / 8);
+        n_ = std::min(all, (grid + 7) / 8);
+        std::unique_lock<std::mutex> lock(d_.m);
+        const uint64_t turn = d_.next++;
+        d_.cv.wait(lock, [&] { return d_.serving == turn && d_.used + n_ <= all; });
+        d_.used += n_;
+        d_.serving++;
+        d_.cv.notify_all();
+    }
+    ~ResidentCus() {
+        std::lock_guard<std::mutex> lock(d_.m);
+        d_.used -= n_;
+        d_.cv.notify_all();
+    }
+    ResidentCus(const ResidentCus &) = delete;
+    ResidentCus &operator=(const ResidentCus &) = delete;
+
+private:
+    struct Device {
+        std::mutex m;
+        std::condition_variable cv;
+        int used = 0;
+        uint64_t next = 0, serving = 0;
+    };
+    static Device &of(int device) {
+        static std::mutex m;
+        static std::map<int, Device> all;
+        std::lock_guard<std::mutex> lock(m);
+        return all[device];
+    }
+    Device &d_;
+    int n_ = 0;
+};
+
+}  // namespace
+
 template <typename T, int D, typename IX, bool NT>
 static int pcg_go(lpm_ctx *c, PcgPlan &P, PcgArgs &a, int64_t maxit, bool *ran) {
     const int M = D == 3 ? 6 : 3;
@@ -665,20 +715,20 @@ static int pcg_go(lpm_ctx *c, PcgPlan &P, PcgArgs &a, int64_t maxit, bool *ran) 
                  hip_done(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device)) &&
                  (int64_t)per * cus >= P.grid;
         P.lds = lds;
+        P.cus = cus;
         P.khz = khz;
     }
     if (!P.fits) return LPM_OK;
     a.wait_ticks = (u64)(c->cg_wait_ms * P.khz);
+    const ResidentCus held(c->device, P.cus, P.grid);  // until the solve has ended
     for (int64_t it = 0;;) {
         hipLaunchKernelGGL(k_pcg_clear, dim3(blocks_for(P.words, 256)), dim3(256), 0, c->stream, P.words,
                            P.slots, c->scal);
         a.it0 = (int)it;
         a.itmax = (int)std::min<int64_t>(it + PCG_LAUNCH_ITERS, 0x7fffffff);
         void *args[] = {&a};
-        const hipError_t e = hipLaunchCooperativeKernel((const void *)kern, dim3(P.grid), dim3(PCG_NT), args, (unsigned)lds,
-                                                        c->stream);
-        if (!hip_done(e)) {  // no cooperative launch here: the caller solves launch by launch
-            P.fits = false;
+        if (!hip_done(hipLaunchKernel((const void *)kern, dim3(P.grid), dim3(PCG_NT), args, lds, c->stream))) {
+            P.fits = false;  // the caller solves launch by launch
             return LPM_OK;
         }
         LPM_HIP(c, hipMemcpyAsync(c->h_scal, c->scal, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, c->stream));

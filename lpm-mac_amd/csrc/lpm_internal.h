@@ -93,7 +93,7 @@ struct PcgPlan {
     const void *kern = nullptr;           // the kernel, the most LDS it may ask for, the LDS that `fits` was found for
     size_t lds_most = 0, lds = 0;
     bool fits = false;                    // its whole grid can be resident
-    int khz = 0;                          // rate of the device's wall clock
+    int cus = 0, khz = 0;                 // CUs of the device, rate of its wall clock
 };
 
 struct lpm_ctx {
