@@ -70,6 +70,7 @@ constexpr int PCG_WG = 256;                 // most workgroups: one per CU
 constexpr int PCG_SPW = 8;                 // most slices of a workgroup: one row per thread
 constexpr int PCG_CZ = 2048;                // most coarse DoFs a workgroup reads
 constexpr int PCG_LA = 64;                  // most aggregates of a workgroup's rows
+constexpr int PCG_SHARES = 32768;           // most shares of P^T r that a workgroup polls
 constexpr int PCG_LAUNCH_ITERS = 1024;      // iterations of one launch (longer solves are continued)
 
 struct PcgArgs {
@@ -551,6 +552,43 @@ static bool hip_done(hipError_t e) {
     return e == hipSuccess;
 }
 
+// Whether neighbouring rows have neighbouring columns: over the rows of eight slices, the groups of 16 particles
+// that the q-th columns of a slice's rows fall into, against the rows (a lattice in its own order 0.1-0.3, a
+// shuffled one 0.9). False when the device could not be read.
+static bool pcg_scattered(lpm_ctx *c, bool *scattered) {
+    constexpr int NS = 8;
+    int32_t ptr[NS][65];
+    int64_t row[NS], rows[NS];
+    for (int k = 0; k < NS; ++k) {
+        row[k] = 64 * (c->nslice * k / NS);
+        rows[k] = std::min<int64_t>(64, c->n - row[k]);
+        if (!hip_done(hipMemcpyAsync(ptr[k], c->cptr + row[k], sizeof(int32_t) * (rows[k] + 1), hipMemcpyDeviceToHost, c->stream)))
+            return false;
+    }
+    if (!hip_done(hipStreamSynchronize(c->stream))) return false;
+    std::vector<int32_t> col[NS];
+    for (int k = 0; k < NS; ++k) {
+        col[k].resize(ptr[k][rows[k]] - ptr[k][0]);
+        if (!col[k].empty() && !hip_done(hipMemcpyAsync(col[k].data(), c->cidx + ptr[k][0], sizeof(int32_t) * col[k].size(),
+                                                        hipMemcpyDeviceToHost, c->stream)))
+            return false;
+    }
+    if (!hip_done(hipStreamSynchronize(c->stream))) return false;
+    int64_t lanes = 0, groups = 0;
+    std::vector<int32_t> g;
+    for (int k = 0; k < NS; ++k)
+        for (int q = 0; q < c->maxconn; ++q) {
+            g.clear();
+            for (int64_t i = 0; i < rows[k]; ++i)
+                if (q < ptr[k][i + 1] - ptr[k][i]) g.push_back(col[k][ptr[k][i] - ptr[k][0] + q] >> 4);
+            lanes += (int64_t)g.size();
+            std::sort(g.begin(), g.end());
+            groups += std::unique(g.begin(), g.end()) - g.begin();
+        }
+    *scattered = 2 * groups > lanes;
+    return true;
+}
+
 // Slots and, for the two-level preconditioner, the rows of each workgroup by aggregate: built once for each of
 // the two kinds and kept, since a caller may switch between them from solve to solve (SC 40^3: 0.5 ms a time).
 // Sets the plan's state: 1 usable, -1 not. No failure in here ends the solve: the launches need none of this.
@@ -610,8 +648,17 @@ static void pcg_prepare(lpm_ctx *c, PcgPlan &P, bool coarse) {
         cnt.assign(c->nagg, 0);
         slot.resize(lagg.size());
         for (size_t q = 0; q < lagg.size(); ++q) slot[q] = cnt[lagg[q]]++;
+        // Where the numbering scatters the rows of a workgroup over many aggregates, every aggregate has shares of
+        // many workgroups, and polling them takes longer than the launches' restriction. Launched against persistent
+        // time by shares: lattices in their own order up to 12,000: 1.08-1.37; shuffled in part or in full: 20,000
+        // to 27,000 1.00-1.23, 32,000 1.05-1.12, 37,000 0.85-0.98, 50,000 0.87, 77,000 0.78, 88,000 0.68-0.70.
+        std::vector<int64_t> upto(c->nagg + 1, 0);
+        for (int g = 0; g < c->nagg; ++g) upto[g + 1] = upto[g] + (int64_t)M * cnt[g];
+        for (int y = 0; y < c->ncoarse; y += per)
+            if (upto[cb[grp[(std::min(c->ncoarse, y + per) - 1) / M] + 1] / M] - upto[cb[grp[y / M]] / M] > PCG_SHARES) return;
         nctr = (int64_t)*std::max_element(cnt.begin(), cnt.end()) * c->ncoarse;
     }
+    if (!c->scol16 && !pcg_scattered(c, &P.scattered)) return;
     P.words = 2 * (nctr + (coarse ? c->ncoarse : 0) + 3 * (int64_t)PCG_SET);
     P.nslot_c = (int)nctr;
     Slab slab;
@@ -758,10 +805,17 @@ int pcg_solve(lpm_ctx *c, int64_t maxit, bool *ran) {
     PcgPlan &P = c->pcg_plan[coarse ? 1 : 0];
     pcg_prepare(c, P, coarse);
     if (P.state != 1) return LPM_OK;
-    PcgArgs a = {};
     const size_t es = c->precision == 0 ? 4 : 8;
     const int D = c->dim;
     const bool idx16 = c->scol16 && c->spmv_idx16;
+    // u is read past the L2s here, an entry of its own for almost every block where the columns are scattered,
+    // while the launched SpMV finds u in them. That costs more than the launches do from 28 MB of such reads per
+    // product on, until at 250 MB the matrix leaves the MALL and its bytes bound both. Launched against persistent
+    // time of shuffled lattices, Jacobi, by MB of u read (MB of matrix): 18 (44) 1.08, 19 (48) 1.12, 25 (63) 1.04, 25 (82)
+    // 1.00, 32 (80) 0.94, 32 (107) 0.95, 35 (79) 0.96, 38 (86) 1.04, 39 (125) 0.87, 49 (156) 0.84, 61 (202) 0.77, 64
+    // (204) 0.80, 66 (209) 0.83; 80 (255) 1.00, 87 (290) 1.09, 88 (280) 1.05, 121 (384) 1.12, 174 (551) 1.11.
+    if (P.scattered && (double)c->nconn * D * es > 28e6 && (double)c->nslots * (D * D * es + 4) < 250e6) return LPM_OK;
+    PcgArgs a = {};
     a.n = c->n;
     a.nslice = c->nslice;
     a.spw = P.spw;

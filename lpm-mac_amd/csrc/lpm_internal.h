@@ -87,6 +87,7 @@ struct PcgPlan {
     int state = 0;                        // 0 not prepared, 1 usable, -1 not
     int spw = 0, grid = 0, nslot_c = 0;   // slices of a workgroup, workgroups, words of one set of coarse shares
     int64_t words = 0;                    // of all slots
+    bool scattered = false;               // neighbouring rows without neighbouring columns
     void *base = nullptr;                 // the one allocation that holds the arrays below
     unsigned long long *slots = nullptr;
     int32_t *lptr = nullptr, *lagg = nullptr, *lslot = nullptr, *lbeg = nullptr, *wpos = nullptr, *cnt = nullptr, *order = nullptr;
