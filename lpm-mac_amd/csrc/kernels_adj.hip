@@ -34,7 +34,6 @@ constexpr int GP = LPM_BOND_GP;
 struct BondGroup {
     int64_t p0;
     int np, B0, nbk;
-    const int *ptr;
 };
 
 __device__ __forceinline__ BondGroup bond_group(int64_t n, const int32_t *__restrict__ bptr, int *sbp, int *own) {
@@ -46,7 +45,6 @@ __device__ __forceinline__ BondGroup bond_group(int64_t n, const int32_t *__rest
     __syncthreads();
     g.B0 = sbp[0];
     g.nbk = sbp[g.np] - g.B0;
-    g.ptr = sbp;
     // eight lanes per particle
     const int p = tid >> 3;
     if (p < g.np)

@@ -17,7 +17,7 @@
 // FP32 (precision 0) or FP64 (precision 1). No host synchronisation happens inside an
 // iteration: the "done" flag makes the remaining kernels of a batch return at once.
 //
-// Vectors are stored padded to VP entries per particle (VP = 4 in 3D, 2 in 2D).
+// Vectors hold VP entries per particle, one for each dimension, without padding.
 #include <algorithm>
 #include <cfloat>
 #include <vector>
