@@ -1269,18 +1269,24 @@ __global__ __launch_bounds__(256) void k_nl_bin(int64_t n, const double *__restr
     atomicAdd(&count[cell], 1);
 }
 
-// Eight lanes per particle over the particles of its 27 cells, three cells in a row being one range of
+// LN lanes per particle over the particles of its 27 cells, three cells in a row being one range of
 // items; the accepted ones take their places by ballot, in any order (k_nl_sort follows). Bound by the gathers
-// of positions, in the caches. A thread per particle ran 729 of them in a chain at SC 41 x 40 x 39
-// (64k particles, lists of 112): count 219 and fill 249 us, now 86 and 93.
-template <bool FILL>
+// of positions, in the caches: by a particle's chain of them while the chip is not full, by their number once
+// it is, and then lanes past the end of a short range are lost. Count and fill in us with a thread, four lanes and
+// eight lanes per particle (items per range):
+//   SC 20^3 (81) 289+353, 70+86, 38+46      SC 64^3 (10) 66+86, 71+79, 85+91      plate of 46,085 (125) 130+148, 51+54, 36+41
+//   SC 36^3 (81) 307+362, 97+104, 68+74     SC 64^3 (28) 177+232, 152+168, 160+171     of 279,720 (8) 24+31, 26+28, 36+37
+//   64k (81) 304+372, 113+126, 91+98        SC 64^3 (81) 425+553, 385+421, 378+397     of 279,720 (125) 269+564, 186+232, 180+205
+//   SC 48^3 (10) 64+72, 33+37, 40+42        FCC 40^3 (40) 326+411, 205+239, 209+224    of 2.1 M (8) 123+238, 173+180, 250+256
+// So eight lanes up to 65,536 particles or from 36 items per range on, else four.
+template <bool FILL, int LN>
 __global__ __launch_bounds__(256) void k_nl_cells(int64_t n, double ratio, const double *__restrict__ xyz,
                                                    const double *__restrict__ L, const int32_t *__restrict__ pcell,
                                                    int64_t nc0, int64_t nc1, int64_t nc2, const int32_t *__restrict__ head,
                                                    const int32_t *__restrict__ items, int32_t *__restrict__ counts,
                                                    const int32_t *__restrict__ nlptr, int32_t *__restrict__ nlidx) {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
-    const int lane = threadIdx.x & 7, group = (threadIdx.x & 63) & ~7;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LN;
+    const int lane = threadIdx.x & (LN - 1), group = (threadIdx.x & 63) & ~(LN - 1);
     if (i >= n) return;
     const double x0 = xyz[3 * i], y0 = xyz[3 * i + 1], z0 = xyz[3 * i + 2], cut = ratio * L[i];
     const int64_t ncs = nc0 * nc1 * nc2, cell = pcell[i];
@@ -1294,7 +1300,7 @@ __global__ __launch_bounds__(256) void k_nl_cells(int64_t n, double ratio, const
             if (y < 0 || z < 0 || y >= nc1 || z >= nc2) continue;
             const int64_t row = layer * ncs + (z * nc1 + y) * nc0;
             const int hi = head[row + xb + 1];
-            for (int t = head[row + xa] + lane; t - lane < hi; t += 8) {  // as often for the eight lanes
+            for (int t = head[row + xa] + lane; t - lane < hi; t += LN) {  // as often for all lanes of a particle
                 int32_t j = 0;
                 bool hit = false;
                 if (t < hi) {
@@ -1302,7 +1308,7 @@ __global__ __launch_bounds__(256) void k_nl_cells(int64_t n, double ratio, const
                     const double dx = x0 - xyz[3 * (int64_t)j], dy = y0 - xyz[3 * (int64_t)j + 1], dz = z0 - xyz[3 * (int64_t)j + 2];
                     hit = sqrt(dx * dx + dy * dy + dz * dz) < cut;
                 }
-                const unsigned m = (unsigned)(__ballot(hit) >> group) & 0xffu;
+                const unsigned m = (unsigned)(__ballot(hit) >> group) & ((1u << LN) - 1);
                 if (FILL && hit) nlidx[o + cnt + __popc(m & ((1u << lane) - 1))] = j;
                 cnt += __popc(m);
             }
@@ -2312,9 +2318,13 @@ static int nonlocal_search_cells(lpm_ctx *c, double ratio, bool *done) {
     hipLaunchKernelGGL(k_cell_fill, dim3(blocks_for(n, 256)), dim3(256), 0, c->stream, n, (const int32_t *)pcell,
                        (const int32_t *)head, count, items);
     if ((rc = check_launch(c, "k_cell_fill"))) { cleanup(); return rc; }
-    hipLaunchKernelGGL((k_nl_cells<false>), dim3(blocks_for(n, 32)), dim3(256), 0, c->stream, n, ratio, (const double *)c->xyz,
-                       (const double *)c->nonlocal_L, (const int32_t *)pcell, nc[0], nc[1], nc[2], (const int32_t *)head,
-                       (const int32_t *)items, counts, (const int32_t *)nullptr, (int32_t *)nullptr);
+    const bool eight = n <= 65536 || 3 * n >= 36 * ncell;
+    auto cells = [&](auto kern, int32_t *cnt, const int32_t *ptr, int32_t *idx) {
+        hipLaunchKernelGGL(kern, dim3(blocks_for(n, eight ? 32 : 64)), dim3(256), 0, c->stream, n, ratio, (const double *)c->xyz,
+                           (const double *)c->nonlocal_L, (const int32_t *)pcell, nc[0], nc[1], nc[2], (const int32_t *)head,
+                           (const int32_t *)items, cnt, ptr, idx);
+    };
+    eight ? cells(k_nl_cells<false, 8>, counts, nullptr, nullptr) : cells(k_nl_cells<false, 4>, counts, nullptr, nullptr);
     if ((rc = check_launch(c, "k_nl_cells(count)"))) { cleanup(); return rc; }
     if (!hip_ok(hipMemcpyAsync(h_cnt.data(), counts, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream), "nonlocal search") ||
         !hip_ok(hipStreamSynchronize(c->stream), "nonlocal search")) { cleanup(); return rc; }
@@ -2337,9 +2347,7 @@ static int nonlocal_search_cells(lpm_ctx *c, double ratio, bool *done) {
         cleanup();
         return rc;
     }
-    hipLaunchKernelGGL((k_nl_cells<true>), dim3(blocks_for(n, 32)), dim3(256), 0, c->stream, n, ratio, (const double *)c->xyz,
-                       (const double *)c->nonlocal_L, (const int32_t *)pcell, nc[0], nc[1], nc[2], (const int32_t *)head,
-                       (const int32_t *)items, counts, (const int32_t *)c->nlptr, c->nlidx);
+    eight ? cells(k_nl_cells<true, 8>, counts, c->nlptr, c->nlidx) : cells(k_nl_cells<true, 4>, counts, c->nlptr, c->nlidx);
     if ((rc = check_launch(c, "k_nl_cells(fill)"))) { cleanup(); return rc; }
     int P = 2;
     while (P < maxlen) P <<= 1;
