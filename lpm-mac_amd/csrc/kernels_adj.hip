@@ -26,8 +26,9 @@ namespace {
 // The four product kernels below are bound by the per-bond arrays they read. As in the force
 // kernels, a workgroup of one wavefront owns LPM_BOND_GP consecutive particles and takes their bonds a
 // lane each, so these reads are contiguous; the per-particle sums then run over values staged in
-// LDS, in bond order. One thread per particle, each walking its own 18 bonds, took 60 + 40 us (J v) and
-// 61 + 78 us (J^T w) at SC 30 x 31 x 29.
+// LDS, in bond order. One thread per particle, each walking its own 18 bonds, took 703 + 460 us (J v) and
+// 922 + 843 us (J^T w) at SC 64^3, now 94 + 107 and 155 + 175; at SC 30 x 31 x 29 60 + 40 and 61 + 78, now 11 + 13 and
+// 18 + 24.
 constexpr int GP = LPM_BOND_GP;
 
 // The particles and bonds of this workgroup; own[t] is the particle rank of bond B0 + t

@@ -43,8 +43,8 @@ __global__ __launch_bounds__(256) void k_dofmask(int64_t n, int dim, const int32
 // Column indices come from the SELL copy (scol: slot c of row i at sp[i/64] + 64 c + i%64); the entries of
 // neighbouring rows are neighbouring threads, so the lanes read few lines, where the CSR list would put
 // every lane on its own. A chain of dependent loads per slot bounds it (column, its aggregate, the
-// block), so what counts is threads in flight: one thread per row, taking its entries in turn, took 218
-// us at BCC 21 x 20 x 19 in FP64 (67 workgroups) and 57 us at SC 12^3.
+// block), so what counts is threads in flight: with one thread per row, taking its entries in turn, SC 64^3 took 633 us
+// (now 250), SC 36^3 in FP64 422 (83), shuffled 535 (100), hex 300 x 340 in FP64 111 (34), BCC 12^3 189 (32).
 template <typename T, int D>
 __global__ __launch_bounds__(64) void k_coarse_rows(int64_t nra, const int32_t *__restrict__ cptr,
                                                      const int32_t *__restrict__ scol, const int64_t *__restrict__ sp,

@@ -6,7 +6,8 @@
 // steps: five kernels of 3-10 us per iteration whose work is a microsecond or two each, and every
 // launch starts with cold caches. Here a workgroup of eight wavefronts owns the same 64-row slices for
 // the whole solve. Its threads hold their rows' x, r, p, s and diagonal in registers, its part of the
-// matrix stays in the XCD's L2, and only these travel between workgroups, once per iteration
+// matrix stays in the XCD's L2 while all of it fits the eight (28 MB; a larger one is streamed past them), and only
+// these travel between workgroups, once per iteration
 // each: the aggregates' shares of P^T r and the coarse correction, the preconditioned residual u (read by the neighbours' SpMV)
 // with the partial sums of (r, u) and (r, r), and the partial sums of (K u, u).
 //
@@ -30,10 +31,13 @@
 // decision, and a result does not depend on scheduling.
 //
 // Time per iteration, launched and here (two-level unless marked; FP32 unless marked):
-//   SC 12^3      25.8 -> 14.2 us      hex 200 x 231   26.8 -> 19.7 us    SC 48^3       66.1 -> 60.9 us
-//   SC 20^3      30.5 -> 17.9 us      hex 350 x 370   35.6 -> 29.3 us    FCC 24^3      46.0 -> 39.1 us
+//   SC 12^3      25.8 -> 14.2 us      hex 200 x 231   26.8 -> 19.7 us    SC 48^3       67.4 -> 61.3 us
+//   SC 20^3      30.5 -> 17.7 us      hex 350 x 370   37.2 -> 29.7 us    FCC 24^3      47.4 -> 38.9 us
 //   SC 28^3      31.7 -> 23.9 us      SC 16^3 Jacobi  18.5 ->  9.6 us    SC 36^3 FP64  63.8 -> 50.8 us
-//   hex 100 x 115, FP64, Jacobi       14.9 -> 9.8 us                     SC 45^3 FP64  90.2 -> 88.9 us
+//   hex 100 x 115, FP64, Jacobi       14.9 -> 9.8 us                     SC 45^3 FP64  91.8 -> 89.4 us
+//   SC 50 x 51 x 51 (130,050)         73.9 -> 65.5 us    in FP64 125 -> 114 us, FP64 Jacobi 112 -> 103 us
+// The bound of 131,072 rows is that of one row per thread. In 3D in FP64 with Jacobi the two come level at 83,000 to
+// 97,000 rows (FCC 27^3 78.1 and 78.4, SC 45^3 77.6 and 80.1, SC 46^3 83.1 and 82.1, BCC 36^3 64.7 and 58.9).
 // Of the 19.7 us at hex 200 x 231 (241 workgroups): shares of P^T r 1.3, waiting for them and Ac^-1 6.6,
 // correction 0.9, u 1.3, its exchange 4.1, SpMV 2.7, its exchange 2.7. Eight wavefronts of up to
 // 256 registers hold a row's state and eight slots in flight; with sixteen of 128 the compiler spilled

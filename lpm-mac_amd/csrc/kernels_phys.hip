@@ -37,7 +37,8 @@ __device__ __forceinline__ double dmin(double a, double b) { return (b < a) ? b 
 // Per-bond work runs lane-per-bond (coalesced loads and stores of the bond arrays); the
 // per-particle sums then run a thread per (particle, sum) over the bond values staged in LDS, in
 // bond order, so every sum is formed in the reference's order. A thread per particle for all its
-// sums left 56 of 64 lanes idle in a serial chain: at FCC 20^3 (32k particles) 15.4 -> 14.3 us here.
+// sums left 56 of 64 lanes idle in a serial chain: SC 64^3 113 -> 110 us, FCC 40^3 117 -> 115, a plate of 400 x 460
+// 56.5 -> 52.6, FCC 20^3 rotated 16.2 -> 15.1, SC 30 x 31 x 29 14.6 -> 13.7.
 constexpr int GP = LPM_BOND_GP;  // particles per workgroup of the bond kernels
 
 __global__ __launch_bounds__(64) void k_geometry_force(
@@ -121,8 +122,8 @@ __global__ __launch_bounds__(64) void k_geometry_force(
 
 // Bond forces only (geometry already current). Bound by memory: six per-bond arrays, read and written in
 // order by the same workgroups as k_geometry_force, a lane per bond. A thread per particle walking its own
-// bonds spread every load over 64 lines: this pass and k_particle_force together 439 -> 101 us at SC 64^3,
-// 39.8 -> 25.3 at FCC 20^3, 14.4 -> 8.4 at a hexagon plate of 1,007 particles.
+// bonds spread every load over 64 lines: SC 64^3 373 -> 38 us, FCC 20^3 rotated 21.1 -> 6.3, a hexagon plate of 1,007
+// particles 10.3 -> 3.5.
 __global__ __launch_bounds__(64) void k_bond_force(int64_t n, int model, const int32_t *__restrict__ bptr,
                                                     const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
                                                     const double *__restrict__ Kn, const double *__restrict__ Tv,
@@ -1094,7 +1095,7 @@ __global__ __launch_bounds__(256) void k_energy_range(int64_t n, const double *_
 // candidate goes into a hash table in LDS, which leaves every id once (SC: 57 of 198 candidates), and the
 // place of an id in the row is the number of smaller ones. Bound by the LDS traffic of the table. A bitonic
 // sort of 512 entries and a scan by 256 threads, which most rows fill to less than half, took 603 us a pass
-// at SC 41 x 40 x 39 (64k particles), now 76.
+// at SC 41 x 40 x 39 (64k particles), now 76; SC 64^3 2433 -> 310, hex 300 x 340 899 -> 78.
 constexpr int PAT_TAB = 2 * LPM_MAXC;  // at most half full, so a probe always ends
 __global__ __launch_bounds__(64) void k_pattern(int64_t n, const int32_t *__restrict__ bptr,
                                                  const int32_t *__restrict__ bsplit, const int32_t *__restrict__ p2,
