@@ -721,8 +721,9 @@ private:
         uint64_t next = 0, serving = 0;
     };
     static Device &of(int device) {
-        static std::mutex m;
-        static std::map<int, Device> all;
+        // never destroyed: a thread may still solve while the process ends
+        static std::mutex &m = *new std::mutex;
+        static std::map<int, Device> &all = *new std::map<int, Device>;
         std::lock_guard<std::mutex> lock(m);
         return all[device];
     }
